@@ -188,6 +188,22 @@ mc_status mc_sddmm_batched(int bits, mc_signedness sign, int layout, int batch, 
                            long long rhs_stride_bytes, int *output_values, long long out_stride, int vec_length,
                            hipStream_t stream);
 
+/* The attention layer's O = half(float(P V) / divisor) for `batch` matrices
+ * sharing one mask: as mc_spmm_batched (signed, default tile) with P read in
+ * the layouts mc_attn_softmax_f16 writes (8-bit [(i/16)][v][16] bytes, 16-bit
+ * [(i/16)][v][low 16][high 16], 4-bit [(i/32)][v][16] nibble pairs),
+ * column_indices not shuffled, and the product divided and rounded to fp16
+ * (round to nearest even) as it is stored: out_f16 row-major [m][n] halves,
+ * matrix b out_stride halves after matrix b - 1 (8-byte aligned, out_stride a
+ * multiple of 4).  (lhs_bits, rhs_bits) is (8, 8), (16, 8), (8, 4) or (4, 4).
+ * Replaces bspmm_8b / _16b8b / _8b4b / _4b
+ * (end2end_eval/sparse_transformer_magicube/src/cuda/deq_spmm.cpp:50-141). */
+mc_status mc_spmm_batched_f16(int lhs_bits, int rhs_bits, int batch, int m_vec, int vec_length, int n, int k,
+                              const int *row_indices, const int *row_offsets, const int *column_indices,
+                              const int *p, long long p_stride_bytes, const int *rhs_matrix,
+                              long long rhs_stride_bytes, float divisor, void *out_f16, long long out_stride,
+                              hipStream_t stream);
+
 /* ---- Quantized sparse attention ------------------------------------------
  * Layer semantics of spMultiheadAttention
  * (end2end_eval/sparse_transformer_magicube/spattention.py:182-216) per

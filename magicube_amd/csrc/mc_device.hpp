@@ -118,6 +118,37 @@ template <typename T> __device__ __forceinline__ T *uniform(T *p) {
     return reinterpret_cast<T *>(((unsigned long long)hi << 32) | lo);
 }
 
+// Division of an int32 accumulator by one launch-wide divisor, rounded as the
+// IEEE quotient float(a) / d.  y = RN(1 / d) from the host, or 0 when d is
+// outside [2^-60, 2^60]: then the kernel divides.  Otherwise q0 = a * y is
+// within 1.5 ulp of the quotient, one correction makes it faithful, and by
+// Markstein's theorem (faithful q, correctly rounded reciprocal) the second
+// gives the correctly rounded quotient: five multiply-adds instead of the
+// division's scale / reciprocal / fix-up sequence.
+struct Divisor {
+    float d;
+    float y;
+};
+inline Divisor make_divisor(float d) {
+    const float m = d < 0.f ? -d : d;
+    return Divisor{d, m >= 0x1p-60f && m <= 0x1p60f ? 1.0f / d : 0.f};
+}
+__device__ __forceinline__ float quotient_fast(float a, float d, float y) {
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-d, q, a), y, q);
+    return __builtin_fmaf(__builtin_fmaf(-d, q, a), y, q);
+}
+// N accumulators divided in place (the branch is uniform: v.y is a launch argument)
+template <int N> __device__ __forceinline__ void divide(const int (&a)[N], const Divisor &v, float (&q)[N]) {
+    if (v.y != 0.f) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = quotient_fast((float)a[i], v.d, v.y);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = (float)a[i] / v.d;
+    }
+}
+
 // Cross-lane read of lane (self + delta) within the wave (delta multiple of 16).
 __device__ __forceinline__ int lane_down(int x, int delta) {
     const int lane = __lane_id();

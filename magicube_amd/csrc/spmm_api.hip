@@ -57,7 +57,7 @@ mc_status spmm_entry(int lhs_bits, int rhs_bits, mc_signedness sign, int config,
                      int k, const int *row_indices, const int *row_offsets, const int *column_indices,
                      const int *values, const int *rhs_matrix, int *output_matrix, hipStream_t stream,
                      int batch = 1, long long values_stride = 0, long long rhs_stride = 0,
-                     long long out_stride = 0) {
+                     long long out_stride = 0, __half *out16 = nullptr, float divisor = 1.f) {
     if (!pair_supported(lhs_bits, rhs_bits)) return MC_EUNSUPPORTED;
     if (batch < 1 || batch > 65535 || values_stride < 0 || rhs_stride < 0 || out_stride < 0) return MC_EINVAL_SHAPE;
     if ((values_stride | rhs_stride) & 3) return MC_EINVAL_SHAPE;   // every matrix starts dword aligned
@@ -70,7 +70,7 @@ mc_status spmm_entry(int lhs_bits, int rhs_bits, mc_signedness sign, int config,
     if (rhs_bytes >= (1LL << 30)) return MC_EINVAL_SHAPE;   // gather offsets stay below 2^30
     if ((long long)m_vec * vec_length * (long long)n >= (1LL << 40)) return MC_EINVAL_SHAPE;
     if (m_vec == 0) return MC_OK;
-    if (!row_offsets || !column_indices || !values || !rhs_matrix || !output_matrix) return MC_EINVAL_ARG;
+    if (!row_offsets || !column_indices || !values || !rhs_matrix || !(output_matrix || out16)) return MC_EINVAL_ARG;
     if (config < -1 || config >= kNumSpmmConfigs) return MC_EINVAL_ARG;
     // a batched launch fills the GPU with (row, tile) x batch workgroups
     int cfg = config >= 0 ? config : default_config(rhs_bits, n, (long long)m_vec * batch);
@@ -100,6 +100,13 @@ mc_status spmm_entry(int lhs_bits, int rhs_bits, mc_signedness sign, int config,
     a.rhs_stride = rhs_stride;
     a.out_stride = out_stride;
     a.batch = batch;
+    if (out16) {
+        // 8-byte stores of four columns
+        if ((reinterpret_cast<uintptr_t>(out16) & 7u) != 0 || (batch > 1 && out_stride % 4 != 0)) return MC_EINVAL_ARG;
+        a.out16 = out16;
+        a.div = make_divisor(divisor);
+        return spmm_layer_launch_pair(lhs_bits, rhs_bits, vec_length, cfg, a, stream);
+    }
     const bool sgn = sign == MC_SIGNED;
     if (lhs_bits == 8 && rhs_bits == 8) return spmm_launch_l8r8(sgn, vec_length, cfg, a, stream);
     if (lhs_bits == 16 && rhs_bits == 8) return spmm_launch_l16r8(sgn, vec_length, cfg, a, stream);
@@ -195,6 +202,19 @@ mc_status mc_spmm_batched(int lhs_bits, int rhs_bits, mc_signedness sign, int co
     return mc::spmm_entry(lhs_bits, rhs_bits, sign, config, m_vec, vec_length, n, k, row_indices, row_offsets,
                           column_indices, values, rhs_matrix, output_matrix, stream, batch, values_stride_bytes,
                           rhs_stride_bytes, out_stride);
+}
+
+mc_status mc_spmm_batched_f16(int lhs_bits, int rhs_bits, int batch, int m_vec, int vec_length, int n, int k,
+                              const int *row_indices, const int *row_offsets, const int *column_indices,
+                              const int *p, long long p_stride_bytes, const int *rhs_matrix,
+                              long long rhs_stride_bytes, float divisor, void *out_f16, long long out_stride,
+                              hipStream_t stream) {
+    if (!((lhs_bits == 8 || lhs_bits == 16) && rhs_bits == 8) && !((lhs_bits == 8 || lhs_bits == 4) && rhs_bits == 4))
+        return MC_EUNSUPPORTED;
+    if (m_vec > 0 && !out_f16) return MC_EINVAL_ARG;
+    return mc::spmm_entry(lhs_bits, rhs_bits, MC_SIGNED, -1, m_vec, vec_length, n, k, row_indices, row_offsets,
+                          column_indices, p, rhs_matrix, nullptr, stream, batch, p_stride_bytes, rhs_stride_bytes,
+                          out_stride, static_cast<__half *>(out_f16), divisor);
 }
 
 }  // extern "C"

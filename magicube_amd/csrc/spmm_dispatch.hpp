@@ -37,7 +37,7 @@ inline bool stationary_fits(int cfg, int n, int k) {
     return c.kind == 1 && n % tb == 0 && (size_t)(k + 1) * tb <= (size_t)kStatLdsBytes;
 }
 
-template <int V, int AB, int BB, bool SGN, int LW, int TPB, int SK, int D, int WPS = 1>
+template <int V, int AB, int BB, bool SGN, int LW, int TPB, int SK, int D, int WPS = 1, bool LAYER = false>
 mc_status spmm_launch_one(SpmmArgs a, hipStream_t stream) {
     constexpr int TILE_N = 16 * LW * (32 / BB);
     if ((a.n / (32 / BB)) % LW != 0) return MC_EUNSUPPORTED;
@@ -46,8 +46,8 @@ mc_status spmm_launch_one(SpmmArgs a, hipStream_t stream) {
     const long long blocks = (long long)a.m_vec * groups;
     if (blocks <= 0) return MC_OK;
     if (blocks > 0x7fffffffLL) return MC_EINVAL_SHAPE;
-    hipLaunchKernelGGL((spmm_kernel<V, AB, BB, SGN, LW, TPB, SK, D, WPS>), dim3((unsigned)blocks, (unsigned)a.batch),
-                       dim3(64 * TPB * SK), 0, stream, a);
+    hipLaunchKernelGGL((spmm_kernel<V, AB, BB, SGN, LW, TPB, SK, D, WPS, LAYER>),
+                       dim3((unsigned)blocks, (unsigned)a.batch), dim3(64 * TPB * SK), 0, stream, a);
     return check_launch();
 }
 
@@ -113,6 +113,32 @@ mc_status spmm_launch_pair(bool sgn, int V, int cfg, const SpmmArgs &a, hipStrea
     }
     return MC_EINVAL_V;
 }
+
+// The attention layer's products (fp16 output, P in the softmax op's layouts):
+// the default tiles of spmm_default_config.
+template <int V, int AB, int BB>
+mc_status spmm_layer_launch_cfg(int cfg, const SpmmArgs &a, hipStream_t s) {
+    switch (cfg) {
+    case 13: return spmm_launch_one<V, AB, BB, true, 1, 8, 1, 1, 1, true>(a, s);
+    case 15: return spmm_launch_one<V, AB, BB, true, 1, 1, 1, 1, 1, true>(a, s);
+    case 16: return spmm_launch_one<V, AB, BB, true, 1, 2, 1, 1, 1, true>(a, s);
+    case 17: return spmm_launch_one<V, AB, BB, true, 1, 4, 1, 1, 1, true>(a, s);
+    case 20: return spmm_launch_one<V, AB, BB, true, 1, 4, 2, 1, 1, true>(a, s);
+    case 22: return spmm_launch_one<V, AB, BB, true, 1, 2, 2, 1, 1, true>(a, s);
+    default: return MC_EUNSUPPORTED;
+    }
+}
+
+template <int AB, int BB> mc_status spmm_layer_launch(int V, int cfg, const SpmmArgs &a, hipStream_t s) {
+    switch (V) {
+    case 2: return spmm_layer_launch_cfg<2, AB, BB>(cfg, a, s);
+    case 4: return spmm_layer_launch_cfg<4, AB, BB>(cfg, a, s);
+    case 8: return spmm_layer_launch_cfg<8, AB, BB>(cfg, a, s);
+    }
+    return MC_EINVAL_V;
+}
+
+mc_status spmm_layer_launch_pair(int lhs_bits, int rhs_bits, int V, int cfg, const SpmmArgs &a, hipStream_t s);
 
 mc_status spmm_launch_l8r8(bool sgn, int V, int cfg, const SpmmArgs &a, hipStream_t s);
 mc_status spmm_launch_l16r8(bool sgn, int V, int cfg, const SpmmArgs &a, hipStream_t s);

@@ -37,6 +37,8 @@
 // The output is the exact sum modulo 2^32.
 #pragma once
 
+#include <hip/hip_fp16.h>
+
 #include "mc_device.hpp"
 
 namespace mc {
@@ -61,7 +63,14 @@ struct SpmmArgs {
     long long rhs_stride;
     long long out_stride;
     int batch;                  // matrices in the launch (gridDim.y), >= 1
+    // attention-layer products (LAYER kernels): half(acc / div) at out16
+    __half *out16;
+    Divisor div;
 };
+
+// Where slot p of an 8-slot group reads its column index when A's 4-bit
+// lanes come as natural nibble pairs: nib_even, then nib_odd of each dword.
+__device__ __forceinline__ int nibble_slot(int p) { return p < 4 ? 2 * p : 2 * p - 7; }
 
 template <int AB, int BB, bool SGN> struct Pair;
 
@@ -134,10 +143,16 @@ struct LdsA {
 
 // A operand of one lane: plane p, vector lane v, reduction slots
 // [slot0, slot0 + 16).  Returns zeros when !ok (buffer offset out of range).
-template <int V, int AB, int BB, bool SGN, class Src>
+// LAYER: A is the quantized softmax's P as that op writes it: 8-bit
+// [(i/16)][v][16] bytes also for 4-bit B, 16-bit [(i/16)][v][low 16][high 16],
+// 4-bit as the reference's SpMM operand.
+template <int V, int AB, int BB, bool SGN, bool LAYER, class Src>
 __device__ __forceinline__ v4i load_a_operand(const Src &va, int slot0, int p, int v, bool ok) {
     const u32 OOB = 0x80000000u;
-    if constexpr (BB != 4) {
+    if constexpr (LAYER && AB == 8) {
+        static_assert(SGN, "P is signed");
+        return va.b128(ok ? (u32)((slot0 >> 4) * 16 * V + 16 * v) : OOB);
+    } else if constexpr (BB != 4) {
         // groups of 16 slots; [V][16] bytes per byte plane
         const int grp = slot0 >> 4;
         if constexpr (AB == 8) {
@@ -154,7 +169,8 @@ __device__ __forceinline__ v4i load_a_operand(const Src &va, int slot0, int p, i
             }
         } else if constexpr (AB == 16) {  // low-byte plane then high-byte plane per group
             const bool hi = SGN ? (p == 0) : (p < 2);
-            const u32 off = ok ? (u32)(grp * 32 * V + (hi ? 16 * V : 0) + 16 * v) : OOB;
+            const u32 off = ok ? (u32)(grp * 32 * V + (LAYER ? 32 * v + (hi ? 16 : 0) : 16 * v + (hi ? 16 * V : 0)))
+                               : OOB;
             v4i x = va.b128(off);
             if (SGN && p == 0) return x;
             const int sh = SGN ? (p == 1 ? 4 : 0) : ((p & 1) == 0 ? 4 : 0);
@@ -236,9 +252,9 @@ __device__ __forceinline__ v4i load_a_operand(const Src &va, int slot0, int p, i
         }
     }
 }
-template <int V, int AB, int BB, bool SGN>
+template <int V, int AB, int BB, bool SGN, bool LAYER = false>
 __device__ __forceinline__ v4i load_a_operand(__amdgpu_buffer_rsrc_t va, int slot0, int p, int v, bool ok) {
-    return load_a_operand<V, AB, BB, SGN>(GlobalA{va}, slot0, p, v, ok);
+    return load_a_operand<V, AB, BB, SGN, LAYER>(GlobalA{va}, slot0, p, v, ok);
 }
 
 template <int LW>
@@ -262,7 +278,13 @@ constexpr int kStageSlots = 1024;
 constexpr u32 kOobAdd = 0x40000000u;
 
 // WPS: waves per SIMD the register allocation must allow (1: no constraint).
-template <int V, int AB, int BB, bool SGN, int LW, int TPB, int SPLITK, int DEPTH, int WPS>
+// LAYER: the attention layer's P V (mc_spmm_batched_f16): A read in the
+// softmax op's layouts and half(acc / div) written, so that neither P nor the
+// int32 product takes a pass of its own.  The int32 round trip and the
+// re-layout were most of these calls: the four layer ops over 12 heads at
+// L = 1960 (8-bit P, 4-bit V) take 126 us instead of 259, over 8 heads at
+// L = 4096 (8-bit P and V) 126 us instead of 136.
+template <int V, int AB, int BB, bool SGN, int LW, int TPB, int SPLITK, int DEPTH, int WPS, bool LAYER = false>
 __global__ __launch_bounds__(64 * TPB * SPLITK) __attribute__((amdgpu_waves_per_eu(WPS))) void spmm_kernel(
     SpmmArgs args) {
     using T = Pair<AB, BB, SGN>;
@@ -390,7 +412,9 @@ __global__ __launch_bounds__(64 * TPB * SPLITK) __attribute__((amdgpu_waves_per_
         for (int i = threadIdx.x; i < cblk * 64; i += NT) {
             u32 o = kOobAdd;
             if (i < cn) {
-                const int idx = args.col_indices[c0 + i];
+                // natural nibble pairs of 4-bit A: the index order moves instead
+                const int slot = LAYER && AB == 4 ? ((c0 + i) & ~7) + nibble_slot((c0 + i) & 7) : c0 + i;
+                const int idx = args.col_indices[slot];
                 if (idx >= 0) o = (u32)idx * row_stride;
             }
             s_off[i] = o;
@@ -423,9 +447,9 @@ __global__ __launch_bounds__(64 * TPB * SPLITK) __attribute__((amdgpu_waves_per_
 #pragma unroll
             for (int t = 0; t < RT; ++t) {
                 if constexpr (kShareA)
-                    ar[t] = load_a_operand<V, AB, BB, SGN>(LdsA{s_a, a_base}, slot0, a_p[t], a_v[t], aok && a_live[t]);
+                    ar[t] = load_a_operand<V, AB, BB, SGN, LAYER>(LdsA{s_a, a_base}, slot0, a_p[t], a_v[t], aok && a_live[t]);
                 else
-                    ar[t] = load_a_operand<V, AB, BB, SGN>(ra, slot0, a_p[t], a_v[t], aok && a_live[t]);
+                    ar[t] = load_a_operand<V, AB, BB, SGN, LAYER>(ra, slot0, a_p[t], a_v[t], aok && a_live[t]);
             }
         };
 
@@ -546,6 +570,27 @@ __global__ __launch_bounds__(64 * TPB * SPLITK) __attribute__((amdgpu_waves_per_
     }
 
     if (!home || !col_ok) return;
+    if constexpr (LAYER) {
+        // read next by the output projection: plain stores
+        __half *const out16 = args.out16 + bz * args.out_stride;
+#pragma unroll
+        for (int i = 0; i < HOME; ++i) {
+            int a[NCOL];
+            float q[NCOL];
+            __half2 h[NCOL / 2];
+#pragma unroll
+            for (int c = 0; c < NCOL; ++c) a[c] = res[c][i];
+            divide<NCOL>(a, args.div, q);
+#pragma unroll
+            for (int c = 0; c < NCOL / 2; ++c) h[c] = __floats2half2_rn(q[2 * c], q[2 * c + 1]);
+            __half *orow = out16 + (size_t)(m * V + 4 * g + i) * (size_t)args.n + (size_t)col_dw * CPD;
+#pragma unroll
+            for (int c = 0; c < NCOL / 2; c += 2)
+                *reinterpret_cast<v2i *>(orow + 2 * c) =
+                    v2i{*reinterpret_cast<const int *>(&h[c]), *reinterpret_cast<const int *>(&h[c + 1])};
+        }
+        return;
+    }
     // lane r owns dwords [col_dw, col_dw + LW): NCOL consecutive columns
 #pragma unroll
     for (int i = 0; i < HOME; ++i) {

@@ -31,11 +31,9 @@ reference feeds its signed quantized Q/K/V to unsigned tensor-core MMAs
 which changes its results wherever a lane is negative; these ops compute the
 signed products the layer means.
 
-4-bit V runs on the library's 4-bit-B SpMM kernels, whose A operand is the
-natural nibble packing with column indices shuffled within groups of 8
-([0, 2, 4, 6, 1, 3, 5, 7], SpMM/SpMM/spmm_benchmark.cpp:204-222): the ops
-shuffle the mask's indices, and re-lay 8-bit P into nibble planes and 16-bit
-P into byte planes, with device tensor ops before the launch.
+Each product is one launch (``mc_spmm_batched_f16``): the kernel reads P as
+the softmax op writes it and the mask's indices in their natural order, and
+divides and rounds to fp16 as it stores.
 """
 from __future__ import annotations
 
@@ -45,8 +43,6 @@ import torch
 
 from . import _lib
 from .attention import bquantization as _bquantization
-
-_SHUFFLE8 = (0, 2, 4, 6, 1, 3, 5, 7)
 
 
 def _ptr(t):
@@ -210,30 +206,6 @@ def q_csr_softmax(row_indices, row_offsets, values, sqrt_dk: float, scale: float
 # deq_spmm.cpp
 # ---------------------------------------------------------------------------
 
-def _shuffled(column_indices: torch.Tensor) -> torch.Tensor:
-    """Column indices shuffled within groups of 8, as the 4-bit-B kernels read them."""
-    if column_indices.numel() % 8:
-        raise ValueError("4-bit V needs the mask aligned to 32 slots")
-    perm = torch.tensor(_SHUFFLE8, dtype=torch.long, device=column_indices.device)
-    return column_indices.view(-1, 8)[:, perm].reshape(-1).contiguous()
-
-
-def _p8_to_nibble_planes(p: torch.Tensor, batch: int, V: int) -> torch.Tensor:
-    """8-bit P [(i/16)][v][16] bytes -> per 32-slot group [low nibbles][V][16
-    bytes] + [high nibbles][V][16 bytes] (the L8-R4 operand)."""
-    b = p.view(torch.uint8).view(batch, -1, 2, V, 16).permute(0, 1, 3, 2, 4).reshape(batch, -1, V, 32)
-    lo, hi = b & 15, b >> 4
-    pack = lambda x: x[..., 0::2] | (x[..., 1::2] << 4)          # noqa: E731
-    return torch.stack([pack(lo), pack(hi)], dim=2).contiguous().view(torch.int32).view(batch, -1)
-
-
-def _p16_to_byte_planes(p: torch.Tensor, batch: int, V: int) -> torch.Tensor:
-    """16-bit P [(i/16)][v][low 16][high 16] -> [(i/16)][low, high][V][16]
-    (the L16-R8 operand)."""
-    b = p.view(torch.uint8).view(batch, -1, V, 2, 16).permute(0, 1, 3, 2, 4)
-    return b.contiguous().view(torch.int32).view(batch, -1)
-
-
 def _bspmm(bits_lhs, bits_rhs, row_indices, row_offsets, column_indices, values, rhs_matrix, vec_length, scale,
            stream):
     _check_v(vec_length)
@@ -251,21 +223,19 @@ def _bspmm(bits_lhs, bits_rhs, row_indices, row_offsets, column_indices, values,
     need = nnz * vec_length * bits_lhs // 8
     if vals.shape[1] * 4 < need:
         raise ValueError(f"values hold {vals.shape[1] * 4} bytes per matrix; the mask needs {need}")
+    # whole groups of the mask's slots: 32 of 4-bit B's (8 of its index
+    # shuffle), 16 of 16-bit P's
+    group = (32 if bits_lhs == 8 else 8) if bits_rhs == 4 else (16 if bits_lhs == 16 else 1)
+    if nnz % group:
+        raise ValueError(f"{bits_lhs}-bit P with {bits_rhs}-bit V needs the mask's slots in groups of "
+                         f"{32 if bits_rhs == 4 else group}, not {nnz}")
     with _on(stream):
-        if bits_rhs == 4:
-            ci = _shuffled(ci)
-        if bits_lhs == 8 and bits_rhs == 4:
-            vals = _p8_to_nibble_planes(vals[:, : need // 4], batch, vec_length)
-        elif bits_lhs == 16:
-            vals = _p16_to_byte_planes(vals[:, : need // 4], batch, vec_length)
         m = m_vec * vec_length
-        acc = torch.empty((batch, m, n), dtype=torch.int32, device=rhs.device)
         out = torch.empty((batch, m, n), dtype=torch.float16, device=rhs.device)
-        lib, st = _lib.lib(), _stream_handle(stream)
-        _lib.check(lib.mc_spmm_batched(bits_lhs, bits_rhs, _lib.MC_SIGNED, -1, batch, m_vec, vec_length, n, k,
-                                       _ptr(ri), _ptr(ro), _ptr(ci), _ptr(vals), vals.stride(0) * 4, _ptr(rhs),
-                                       k * n_int32 * 4, _ptr(acc), m * n, st), f"bspmm L{bits_lhs}-R{bits_rhs}")
-        _lib.check(lib.mc_attn_dequant_f16(_ptr(acc), acc.numel(), float(scale), _ptr(out), st), "bspmm dequant")
+        _lib.check(_lib.lib().mc_spmm_batched_f16(bits_lhs, bits_rhs, batch, m_vec, vec_length, n, k, _ptr(ri),
+                                                  _ptr(ro), _ptr(ci), _ptr(vals), vals.stride(0) * 4, _ptr(rhs),
+                                                  k * n_int32 * 4, float(scale), _ptr(out), m * n,
+                                                  _stream_handle(stream)), f"bspmm L{bits_lhs}-R{bits_rhs}")
     return out
 
 
