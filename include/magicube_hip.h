@@ -188,6 +188,21 @@ mc_status mc_sddmm_batched(int bits, mc_signedness sign, int layout, int batch, 
                            long long rhs_stride_bytes, int *output_values, long long out_stride, int vec_length,
                            hipStream_t stream);
 
+/* The attention layer's logits half(float(S) / divisor) for `batch` matrices
+ * sharing one mask: as mc_sddmm_batched (signed, vector-major [slot][v]) with
+ * the products divided and rounded to fp16 (round to nearest even) as they
+ * are stored, and every other slot of [0, slots) set to 0.  bits 8 or 4,
+ * k <= 512 (MC_EUNSUPPORTED beyond: use mc_sddmm_batched and
+ * mc_attn_dequant_f16).  row_indices is a permutation of the rows; out_f16
+ * 8-byte aligned, matrix b out_stride halves after matrix b - 1.
+ * Replaces bsddmm_8b / _4b
+ * (end2end_eval/sparse_transformer_magicube/src/cuda/deq_sddmm.cpp:56-93). */
+mc_status mc_sddmm_batched_f16(int bits, int batch, int m_vec, int k, int n, const int *row_indices,
+                               const int *row_offsets, const int *col_indices, int slots, const int *lhs_matrix,
+                               long long lhs_stride_bytes, const int *rhs_matrix, long long rhs_stride_bytes,
+                               float divisor, void *out_f16, long long out_stride, int vec_length,
+                               hipStream_t stream);
+
 /* The attention layer's O = half(float(P V) / divisor) for `batch` matrices
  * sharing one mask: as mc_spmm_batched (signed, default tile) with P read in
  * the layouts mc_attn_softmax_f16 writes (8-bit [(i/16)][v][16] bytes, 16-bit

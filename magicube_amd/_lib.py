@@ -57,6 +57,7 @@ _SIGS["mc_layernorm_f16"] = (_I, [_LL, _I, _P, _P, _P, _P, _F, _P, _P])
 _SIGS["mc_attn_softmax_f16"] = (_I, [_I, _I, _I, _P, _P, _P, _LL, _F, _F, _I, _P, _LL, _P])
 _SIGS["mc_spmm_batched"] = (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _LL, _P, _LL, _P, _LL, _P])
 _SIGS["mc_spmm_batched_f16"] = (_I, [_I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _LL, _P, _LL, _F, _P, _LL, _P])
+_SIGS["mc_sddmm_batched_f16"] = (_I, [_I, _I, _I, _I, _I, _P, _P, _P, _I, _P, _LL, _P, _LL, _F, _P, _LL, _I, _P])
 _SIGS["mc_sddmm_batched"] = (_I, [_I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _LL, _P, _LL, _P, _LL, _I, _P])
 for _name in ("mc_spmm_l8r8", "mc_spmm_l16r8", "mc_spmm_l8r4", "mc_spmm_l4r4", "mc_spmm_l12r8", "mc_spmm_l16r16",
               "mc_spmm_l12r4", "mc_spmm_l16r4"):

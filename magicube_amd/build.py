@@ -40,6 +40,7 @@ LIB_SOURCES = [
     "spmm_l12r4.hip",
     "spmm_l16r4.hip",
     "spmm_layer.hip",
+    "gaps.hip",
 ]
 OPTIONAL_SOURCES = ["sddmm.hip", "attention.hip", "layernorm.hip"]
 # Vendor-library comparators (rocSPARSE, hipBLASLt): a library of their own so

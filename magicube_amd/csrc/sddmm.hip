@@ -11,32 +11,32 @@ namespace {
 // more of the row's A operands per wave.  Measured on MI355X at
 // M = N = 4096, V = 8: K = 64 5 % faster with 16 waves, K = 128 and 512
 // 7-11 % slower.
-template <int V, int BITS, bool SGN, int NKC, bool REF>
+template <int V, int BITS, bool SGN, int NKC, int OUT>
 mc_status sddmm_launch(const SddmmArgs &a, int batch, hipStream_t s) {
     constexpr int W = NKC == 1 ? 16 : 8;
     constexpr int TPW = NKC == 1 ? 1 : (NKC >= 4 ? 1 : 4 / NKC);
-    hipLaunchKernelGGL((sddmm_kernel<V, BITS, SGN, NKC, W, TPW, REF>), dim3((unsigned)a.m_vec, (unsigned)batch),
+    hipLaunchKernelGGL((sddmm_kernel<V, BITS, SGN, NKC, W, TPW, OUT>), dim3((unsigned)a.m_vec, (unsigned)batch),
                        dim3(64 * W), 0, s, a);
     return check_launch();
 }
 
-template <int V, int BITS, bool SGN, bool REF>
+template <int V, int BITS, bool SGN, int OUT>
 mc_status sddmm_launch_k(int nkc, const SddmmArgs &a, int batch, hipStream_t s) {
     switch (nkc) {
-    case 1: return sddmm_launch<V, BITS, SGN, 1, REF>(a, batch, s);
-    case 2: return sddmm_launch<V, BITS, SGN, 2, REF>(a, batch, s);
-    case 4: return sddmm_launch<V, BITS, SGN, 4, REF>(a, batch, s);
-    case 8: return sddmm_launch<V, BITS, SGN, 8, REF>(a, batch, s);
+    case 1: return sddmm_launch<V, BITS, SGN, 1, OUT>(a, batch, s);
+    case 2: return sddmm_launch<V, BITS, SGN, 2, OUT>(a, batch, s);
+    case 4: return sddmm_launch<V, BITS, SGN, 4, OUT>(a, batch, s);
+    case 8: return sddmm_launch<V, BITS, SGN, 8, OUT>(a, batch, s);
     default: return MC_EUNSUPPORTED;
     }
 }
 
-template <int BITS, bool SGN, bool REF>
+template <int BITS, bool SGN, int OUT>
 mc_status sddmm_launch_v(int V, int nkc, const SddmmArgs &a, int batch, hipStream_t s) {
     switch (V) {
-    case 2: return sddmm_launch_k<2, BITS, SGN, REF>(nkc, a, batch, s);
-    case 4: return sddmm_launch_k<4, BITS, SGN, REF>(nkc, a, batch, s);
-    case 8: return sddmm_launch_k<8, BITS, SGN, REF>(nkc, a, batch, s);
+    case 2: return sddmm_launch_k<2, BITS, SGN, OUT>(nkc, a, batch, s);
+    case 4: return sddmm_launch_k<4, BITS, SGN, OUT>(nkc, a, batch, s);
+    case 8: return sddmm_launch_k<8, BITS, SGN, OUT>(nkc, a, batch, s);
     default: return MC_EINVAL_V;
     }
 }
@@ -44,16 +44,17 @@ mc_status sddmm_launch_v(int V, int nkc, const SddmmArgs &a, int batch, hipStrea
 template <int BITS>
 mc_status sddmm_launch_all(bool sgn, bool ref, int V, int nkc, const SddmmArgs &a, int batch, hipStream_t s) {
     if (sgn)
-        return ref ? sddmm_launch_v<BITS, true, true>(V, nkc, a, batch, s)
-                   : sddmm_launch_v<BITS, true, false>(V, nkc, a, batch, s);
-    return ref ? sddmm_launch_v<BITS, false, true>(V, nkc, a, batch, s)
-               : sddmm_launch_v<BITS, false, false>(V, nkc, a, batch, s);
+        return ref ? sddmm_launch_v<BITS, true, kOutReference>(V, nkc, a, batch, s)
+                   : sddmm_launch_v<BITS, true, kOutVector>(V, nkc, a, batch, s);
+    return ref ? sddmm_launch_v<BITS, false, kOutReference>(V, nkc, a, batch, s)
+               : sddmm_launch_v<BITS, false, kOutVector>(V, nkc, a, batch, s);
 }
 
 mc_status sddmm_entry(int bits, mc_signedness sign, int layout, int m_vec, int k, int n, const int *row_indices,
                       const int *row_offsets, const int *col_indices, const int *lhs_matrix, const int *rhs_matrix,
                       int *output_values, int vec_length, hipStream_t stream, int batch = 1,
-                      long long lhs_stride = 0, long long rhs_stride = 0, long long out_stride = 0) {
+                      long long lhs_stride = 0, long long rhs_stride = 0, long long out_stride = 0,
+                      __half *out16 = nullptr, float divisor = 1.f, int slots = 0) {
     if (batch < 1 || batch > 65535 || lhs_stride < 0 || rhs_stride < 0 || out_stride < 0) return MC_EINVAL_SHAPE;
     if ((lhs_stride | rhs_stride) & 3) return MC_EINVAL_SHAPE;   // every matrix starts dword aligned
     if (bits != 16 && bits != 8 && bits != 4) return MC_EUNSUPPORTED;
@@ -69,7 +70,7 @@ mc_status sddmm_entry(int bits, mc_signedness sign, int layout, int m_vec, int k
     const long long rhs_bytes = (long long)n * k * bits / 8;
     if (lhs_bytes >= (1LL << 30) || rhs_bytes >= (1LL << 30)) return MC_EINVAL_SHAPE;
     if (m_vec == 0) return MC_OK;
-    if (!row_offsets || !col_indices || !lhs_matrix || !rhs_matrix || !output_values) return MC_EINVAL_ARG;
+    if (!row_offsets || !col_indices || !lhs_matrix || !rhs_matrix || !(output_values || out16)) return MC_EINVAL_ARG;
     SddmmArgs a{};
     a.m_vec = m_vec;
     a.k = k;
@@ -85,6 +86,20 @@ mc_status sddmm_entry(int bits, mc_signedness sign, int layout, int m_vec, int k
     a.lhs_stride = lhs_stride;
     a.rhs_stride = rhs_stride;
     a.out_stride = out_stride;
+    if (out16) {
+        if (k > 512 || bits == 16) return MC_EUNSUPPORTED;   // one pass over K
+        // a lane's rows of a slot are stored together: 8 bytes, 4 at V = 2
+        const long long unit = vec_length == 2 ? 4 : 8;
+        if ((reinterpret_cast<uintptr_t>(out16) | (unsigned long long)(batch > 1 ? 2 * out_stride : 0)) & (unit - 1))
+            return MC_EINVAL_ARG;
+        a.out16 = out16;
+        a.div = make_divisor(divisor);
+        const mc_status st = zero_gaps(batch, m_vec, row_offsets, slots, 8, 16 * vec_length, out16, 2 * out_stride,
+                                       stream);
+        if (st != MC_OK) return st;
+        return bits == 8 ? sddmm_launch_v<8, true, kOutHalf>(vec_length, nkc, a, batch, stream)
+                         : sddmm_launch_v<4, true, kOutHalf>(vec_length, nkc, a, batch, stream);
+    }
     const bool sgn = sign == MC_SIGNED, ref = layout == MC_SDDMM_OUT_REFERENCE;
     if (bits == 16) return sddmm_launch_all<16>(sgn, ref, vec_length, nkc, a, batch, stream);
     return bits == 8 ? sddmm_launch_all<8>(sgn, ref, vec_length, nkc, a, batch, stream)
@@ -132,6 +147,18 @@ mc_status mc_sddmm_batched(int bits, mc_signedness sign, int layout, int batch, 
     return mc::sddmm_entry(bits, sign, layout, m_vec, k, n, row_indices, row_offsets, col_indices, lhs_matrix,
                            rhs_matrix, output_values, vec_length, stream, batch, lhs_stride_bytes,
                            rhs_stride_bytes, out_stride);
+}
+
+mc_status mc_sddmm_batched_f16(int bits, int batch, int m_vec, int k, int n, const int *row_indices,
+                               const int *row_offsets, const int *col_indices, int slots, const int *lhs_matrix,
+                               long long lhs_stride_bytes, const int *rhs_matrix, long long rhs_stride_bytes,
+                               float divisor, void *out_f16, long long out_stride, int vec_length,
+                               hipStream_t stream) {
+    if (slots < 0) return MC_EINVAL_SHAPE;
+    if (m_vec > 0 && !out_f16) return MC_EINVAL_ARG;
+    return mc::sddmm_entry(bits, MC_SIGNED, MC_SDDMM_OUT_VECTOR, m_vec, k, n, row_indices, row_offsets, col_indices,
+                           lhs_matrix, rhs_matrix, nullptr, vec_length, stream, batch, lhs_stride_bytes,
+                           rhs_stride_bytes, out_stride, static_cast<__half *>(out_f16), divisor, slots);
 }
 
 }  // extern "C"

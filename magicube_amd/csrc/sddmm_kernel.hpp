@@ -29,6 +29,8 @@
 // vector-major [j][v].
 #pragma once
 
+#include <hip/hip_fp16.h>
+
 #include "mc_device.hpp"
 
 namespace mc {
@@ -51,7 +53,15 @@ struct SddmmArgs {
     long long lhs_stride;
     long long rhs_stride;
     long long out_stride;
+    // kOutHalf: half(sum / div) at out16 (strides in halves)
+    __half *out16;
+    Divisor div;
 };
+
+// Output of a slot: int32 in the reference layout [(j/8)][v][j%8] or
+// vector-major [j][v], or fp16 vector-major divided by args.div (the
+// attention layer's logits, K in one pass; see sddmm.hip for what it saves).
+constexpr int kOutReference = 0, kOutVector = 1, kOutHalf = 2;
 
 template <int BITS, bool SGN> struct SddmmDigits;
 template <bool SGN> struct SddmmDigits<8, SGN> {
@@ -103,9 +113,10 @@ __device__ __forceinline__ v4i expand_nibbles(v4i x, bool sext, u32 xor_mask) {
 
 constexpr u32 kSddmmOob = 0x40000000u;
 
-template <int V, int BITS, bool SGN, int NKC, int W, int TPW, bool OUT_REF>
+template <int V, int BITS, bool SGN, int NKC, int W, int TPW, int OUT>
 __global__ __launch_bounds__(64 * W) void sddmm_kernel(SddmmArgs args) {
     using D = SddmmDigits<BITS, SGN>;
+    constexpr bool OUT_REF = OUT == kOutReference;
     constexpr int P = D::P;
     constexpr int ROWS = P * V;
     constexpr int OB = D::OB;
@@ -282,6 +293,22 @@ __global__ __launch_bounds__(64 * W) void sddmm_kernel(SddmmArgs args) {
 #pragma unroll
                         for (int i = 0; i < 4; ++i) tq[i] = j < end ? res[i] : 0;
                         quad_transpose4(tq, lane);
+                    }
+                    if constexpr (OUT == kOutHalf) {
+                        if (g < (V + 3) / 4 && tg + t < ctiles && j < wend) {
+                            float q[HOME];
+                            int a[HOME];
+#pragma unroll
+                            for (int i = 0; i < HOME; ++i) a[i] = j < end ? res[i] : 0;
+                            divide<HOME>(a, args.div, q);
+                            __half2 h[HOME / 2];
+#pragma unroll
+                            for (int i = 0; i < HOME / 2; ++i) h[i] = __floats2half2_rn(j < end ? q[2 * i] : 0.f, j < end ? q[2 * i + 1] : 0.f);
+                            int *o = reinterpret_cast<int *>(args.out16 + bz * args.out_stride + (size_t)j * V + 4 * g);
+                            if constexpr (HOME == 4) *reinterpret_cast<v2i *>(o) = v2i{*reinterpret_cast<const int *>(&h[0]), *reinterpret_cast<const int *>(&h[1])};
+                            else *o = *reinterpret_cast<const int *>(&h[0]);
+                        }
+                        continue;
                     }
                     if (g < (V + 3) / 4 && tg + t < ctiles && j < wend) {
                         auto store_each = [&]() {

@@ -126,10 +126,15 @@ def _bsddmm(bits, row_indices, row_offsets, column_indices, lhs_matrix, rhs_matr
         raise ValueError(f"lhs_matrix has {m} rows; the mask covers {m_vec} vector rows of {vec_length}")
     nnz = ci.numel()
     with _on(stream):
-        acc = torch.zeros((batch, nnz * vec_length), dtype=torch.int32, device=lhs.device)
         out = torch.empty((batch, nnz * vec_length) if batched else (nnz * vec_length,), dtype=torch.float16,
                           device=lhs.device)
         lib, st = _lib.lib(), _stream_handle(stream)
+        if k <= 512 and m_vec:        # K in one pass: the kernel stores fp16 itself
+            _lib.check(lib.mc_sddmm_batched_f16(bits, batch, m_vec, k, n, _ptr(ri), _ptr(ro), _ptr(ci), nnz,
+                                                _ptr(lhs), m * k_int32 * 4, _ptr(rhs), n * k_int32 * 4, float(scale),
+                                                _ptr(out), nnz * vec_length, vec_length, st), f"bsddmm_{bits}b")
+            return out
+        acc = torch.zeros((batch, nnz * vec_length), dtype=torch.int32, device=lhs.device)
         _lib.check(lib.mc_sddmm_batched(bits, _lib.MC_SIGNED, 1, batch, m_vec, k, n, _ptr(ri), _ptr(ro), _ptr(ci),
                                         _ptr(lhs), m * k_int32 * 4, _ptr(rhs), n * k_int32 * 4, _ptr(acc),
                                         nnz * vec_length, vec_length, st), f"bsddmm_{bits}b")

@@ -57,3 +57,39 @@ def test_bspmm_edges(pair, V, n, divisor):
     with np.errstate(over="ignore"):
         exp = oatt.ref_bspmm(P, v, pairs, cols, V, divisor)
     assert np.array_equal(bits16(out), exp.view(np.uint16))
+
+
+def scattered(pairs, cols, seed):
+    """The same rows laid out in another order, with gaps before, between and after them."""
+    rng = np.random.default_rng(seed)
+    rows = pairs.size // 2
+    where, at = np.zeros_like(pairs), 32
+    out = np.full(2 * cols.size + 32 * (rows + 2), -1, np.int32)
+    for i in rng.permutation(rows):
+        n = int(pairs[2 * i + 1] - pairs[2 * i])
+        where[2 * i:2 * i + 2] = at, at + n
+        out[at:at + n] = cols[pairs[2 * i]:pairs[2 * i + 1]]
+        at += (n + 31) // 32 * 32 + 32 * int(rng.integers(0, 2))
+    return where, out[:at + 32]
+
+
+@pytest.mark.parametrize("bits,k", [(8, 64), (4, 64), (8, 192), (4, 512), (8, 576)])
+@pytest.mark.parametrize("V", [8, 4, 2])
+@pytest.mark.parametrize("layout", ["aligned", "scattered"])
+def test_bsddmm_edges(bits, k, V, layout):
+    batch, divisor = 2, 1296.0 if k == 64 else 7.3
+    order, pairs, cols = ragged_mask(32 if bits == 4 else 16, seed=V + k)
+    if layout == "scattered":
+        pairs, cols = scattered(pairs, cols, seed=k)
+    rng = np.random.default_rng(k + V)
+    lo, hi = -(1 << (bits - 1)), 1 << (bits - 1)
+    lhs = rng.integers(lo, hi, size=(batch, len(COUNTS) * V, k))
+    rhs = rng.integers(lo, hi, size=(batch, KEYS, k))
+    # memory that the op must overwrite or zero
+    torch.full((batch * cols.size * V,), float("nan"), dtype=torch.float16, device="cuda")
+    fn = sptrans.bsddmm_8b if bits == 8 else sptrans.bsddmm_4b
+    print(f"bsddmm bits={bits} k={k} V={V} {layout}", flush=True)
+    got = fn(dev(order), dev(pairs), dev(cols), packed(lhs, bits), packed(rhs, bits), V, bits, divisor)
+    torch.cuda.synchronize()
+    exp = oatt.ref_bsddmm(lhs, rhs, pairs, cols, V, divisor)
+    assert np.array_equal(bits16(got), exp.view(np.uint16))
