@@ -192,8 +192,8 @@ mc_status mc_sddmm_batched(int bits, mc_signedness sign, int layout, int batch, 
  * sharing one mask: as mc_sddmm_batched (signed, vector-major [slot][v]) with
  * the products divided and rounded to fp16 (round to nearest even) as they
  * are stored, and every other slot of [0, slots) set to 0.  bits 8 or 4,
- * k <= 512 (MC_EUNSUPPORTED beyond: use mc_sddmm_batched and
- * mc_attn_dequant_f16).  row_indices is a permutation of the rows; out_f16
+ * k <= 512, 2^-60 <= |divisor| <= 2^60 (MC_EUNSUPPORTED beyond: use
+ * mc_sddmm_batched and mc_attn_dequant_f16).  row_indices is a permutation of the rows; out_f16
  * 8-byte aligned, matrix b out_stride halves after matrix b - 1.
  * Replaces bsddmm_8b / _4b
  * (end2end_eval/sparse_transformer_magicube/src/cuda/deq_sddmm.cpp:56-93). */

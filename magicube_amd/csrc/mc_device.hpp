@@ -136,7 +136,12 @@ inline Divisor make_divisor(float d) {
 __device__ __forceinline__ float quotient_fast(float a, float d, float y) {
     float q = a * y;
     q = __builtin_fmaf(__builtin_fmaf(-d, q, a), y, q);
-    return __builtin_fmaf(__builtin_fmaf(-d, q, a), y, q);
+    q = __builtin_fmaf(__builtin_fmaf(-d, q, a), y, q);
+    // the fp32 quotient is a result of its own: without this the compiler
+    // folds a following conversion to fp16 into the last step
+    // (v_fma_mixlo_f16), which rounds once and differs at ties
+    asm("" : "+v"(q));
+    return q;
 }
 // N accumulators divided in place (the branch is uniform: v.y is a launch argument)
 template <int N> __device__ __forceinline__ void divide(const int (&a)[N], const Divisor &v, float (&q)[N]) {

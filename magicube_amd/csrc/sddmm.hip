@@ -5,19 +5,39 @@
 namespace mc {
 namespace {
 
-// One workgroup per vector row.  A single 64-deep chunk (K = 64) gives each
-// of 16 waves one 16-slot tile at a time, so a row's gathers are spread over
-// more waves; deeper K keeps 8 waves with up to four tiles each, which hold
-// more of the row's A operands per wave.  Measured on MI355X at
-// M = N = 4096, V = 8: K = 64 5 % faster with 16 waves, K = 128 and 512
-// 7-11 % slower.
+constexpr int kMaxWaves = 8;   // waves per row
+
+// Waves per row W and tiles per group T.  Under 1024 rows (times the batch) a
+// launch is one round of workgroups, so a row is spread over more waves and,
+// at K <= 128, single tiles; from there on fewer waves with longer pipelines
+// keep more rows resident.  Measured on MI355X, us (rows x N, K, sparsity):
+//                            W8 T1   W8 T2   W4 T1   W4 T2   W2 T2   W16 T1
+//   512 x 4096, 64, 0.9        4.9     5.0     5.7     5.6     7.3     5.6
+//   512 x 4096, 128, 0.9       5.4     5.6     6.1     6.1     7.8     6.6
+//   256 x 2304, 512, 0.9       5.8     5.3     6.2     6.0     7.0     (8 at most)
+//   1024 x 8192, 64, 0.9      11.6    11.1    11.2    10.6    13.2    13.0
+//   1024 x 8192, 128, 0.9     13.5    12.8    12.8    12.4    14.7    15.5
+//   1024 x 8192, 512, 0.9     35.9    28.6    30.9    26.7    28.7
+// against 5.1, 7.0, 7.7, 11.7, 18.7 and 54.3 for 16 (K = 64) or 8 waves with
+// gathers in the operand layout and nothing in flight across groups.  16-bit
+// operands (two digits) keep one tile: 10.8 against 11.3 at K = 512.
+template <int V, int BITS, bool SGN, int NKC, int TPW, int OUT>
+mc_status sddmm_launch_tiles(const SddmmArgs &a, int waves, int batch, hipStream_t s) {
+    hipLaunchKernelGGL((sddmm_kernel<V, BITS, SGN, NKC, TPW, kMaxWaves, OUT>), dim3((unsigned)a.m_vec, (unsigned)batch),
+                       dim3(64 * waves), 0, s, a);
+    return check_launch();
+}
+
 template <int V, int BITS, bool SGN, int NKC, int OUT>
 mc_status sddmm_launch(const SddmmArgs &a, int batch, hipStream_t s) {
-    constexpr int W = NKC == 1 ? 16 : 8;
-    constexpr int TPW = NKC == 1 ? 1 : (NKC >= 4 ? 1 : 4 / NKC);
-    hipLaunchKernelGGL((sddmm_kernel<V, BITS, SGN, NKC, W, TPW, OUT>), dim3((unsigned)a.m_vec, (unsigned)batch),
-                       dim3(64 * W), 0, s, a);
-    return check_launch();
+    const bool one_round = (long long)a.m_vec * batch < 1024;
+    const int waves = one_round ? 8 : 4;
+    if constexpr (BITS == 16) {
+        return sddmm_launch_tiles<V, BITS, SGN, NKC, 1, OUT>(a, waves, batch, s);
+    } else if constexpr (NKC <= 2) {
+        if (one_round) return sddmm_launch_tiles<V, BITS, SGN, NKC, 1, OUT>(a, waves, batch, s);
+    }
+    if constexpr (BITS != 16) return sddmm_launch_tiles<V, BITS, SGN, NKC, 2, OUT>(a, waves, batch, s);
 }
 
 template <int V, int BITS, bool SGN, int OUT>
@@ -94,6 +114,7 @@ mc_status sddmm_entry(int bits, mc_signedness sign, int layout, int m_vec, int k
             return MC_EINVAL_ARG;
         a.out16 = out16;
         a.div = make_divisor(divisor);
+        if (a.div.y == 0.f) return MC_EUNSUPPORTED;
         const mc_status st = zero_gaps(batch, m_vec, row_offsets, slots, 8, 16 * vec_length, out16, 2 * out_stride,
                                        stream);
         if (st != MC_OK) return st;

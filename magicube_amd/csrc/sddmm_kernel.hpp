@@ -79,16 +79,19 @@ template <bool SGN> struct SddmmDigits<16, SGN> {
 
 // 16 k-values of 16-bit lanes at off_bytes as two byte-digit operands
 // (k order kept): hi = high bytes, lo = low bytes, each XORed with its mask.
-__device__ __forceinline__ void load_k16_w16(__amdgpu_buffer_rsrc_t r, u32 off_bytes, u32 xhi, u32 xlo, v4i &hi,
-                                             v4i &lo) {
-    const v4i w0 = buf_load_b128(r, off_bytes);
-    const v4i w1 = buf_load_b128(r, off_bytes + 16u);
+__device__ __forceinline__ void split_w16(v4i w0, v4i w1, u32 xhi, u32 xlo, v4i &hi, v4i &lo) {
     const u32 w[8] = {(u32)w0[0], (u32)w0[1], (u32)w0[2], (u32)w0[3], (u32)w1[0], (u32)w1[1], (u32)w1[2], (u32)w1[3]};
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         hi[q] = (int)(perm(w[2 * q + 1], w[2 * q], 0x07050301u) ^ xhi);
         lo[q] = (int)(perm(w[2 * q + 1], w[2 * q], 0x06040200u) ^ xlo);
     }
+}
+__device__ __forceinline__ void load_k16_w16(__amdgpu_buffer_rsrc_t r, u32 off_bytes, u32 xhi, u32 xlo, v4i &hi,
+                                             v4i &lo) {
+    const v4i w0 = buf_load_b128(r, off_bytes);
+    const v4i w1 = buf_load_b128(r, off_bytes + 16u);
+    split_w16(w0, w1, xhi, xlo, hi, lo);
 }
 
 // 16 k-values of one packed row at k offset k0 (multiple of 16) as an int8
@@ -113,14 +116,31 @@ __device__ __forceinline__ v4i expand_nibbles(v4i x, bool sext, u32 xor_mask) {
 
 constexpr u32 kSddmmOob = 0x40000000u;
 
-template <int V, int BITS, bool SGN, int NKC, int W, int TPW, int OUT>
-__global__ __launch_bounds__(64 * W) void sddmm_kernel(SddmmArgs args) {
+// Gathered rhs rows arrive row-contiguous: lane 4i + j holds piece j of row
+// i, so that a load touches each row's line once (16 L1 accesses for 16 rows;
+// loaded in the operand layout, 16 lanes of 16 rows at a time, the same load
+// makes 64).  One ds_bpermute per dword moves them to the operand layout,
+// lane (r, g) <- lane 4r + g (addr = 4 (4r + g)).
+template <int N = 4> __device__ __forceinline__ v4i row_to_operand(v4i x, int addr) {
+#pragma unroll
+    for (int q = 0; q < N; ++q) x[q] = __builtin_amdgcn_ds_bpermute(addr, x[q]);
+    return x;
+}
+
+// W waves per row (blockDim.x / 64); wave w takes groups of TPW 16-slot tiles
+// w, w + W, ...  A wave's loads run ahead of its arithmetic: while a group is
+// multiplied and stored, the next group's gathers are in flight (issued before
+// the stores, since a wait for a load also waits for older stores) and the
+// column indices of the group after that.
+template <int V, int BITS, bool SGN, int NKC, int TPW, int MAXW, int OUT>
+__global__ __launch_bounds__(64 * MAXW) void sddmm_kernel(SddmmArgs args) {
     using D = SddmmDigits<BITS, SGN>;
     constexpr bool OUT_REF = OUT == kOutReference;
     constexpr int P = D::P;
     constexpr int ROWS = P * V;
     constexpr int OB = D::OB;
     constexpr bool W16 = BITS == 16;
+    constexpr int BD = W16 ? 2 : 1;            // rhs digits (16-bit: low, high)
     // 16-bit digit masks: unsigned bytes and signed low bytes become b ^ 0x80
     constexpr u32 XHI = SGN ? 0u : 0x80808080u, XLO = 0x80808080u;
     constexpr int HOME = V < 4 ? V : 4;
@@ -128,16 +148,20 @@ __global__ __launch_bounds__(64 * W) void sddmm_kernel(SddmmArgs args) {
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int W = (int)blockDim.x >> 6;
     const int r = lane & 15, g = lane >> 4;
     const int m = uniform(args.row_indices ? args.row_indices[blockIdx.x] : (int)blockIdx.x);
     const int start = uniform(args.row_offsets[2 * m]);
     const int end = uniform(args.row_offsets[2 * m + 1]);
     const int wend = start + ((end - start + 7) & ~7);   // written slots
+    const int ctiles = (wend - start + 15) >> 4;
+    const int step = W * TPW;
 
     const u32 row_bytes = (u32)args.k * BITS / 8;
     const long long bz = blockIdx.y;
     const __amdgpu_buffer_rsrc_t rl = make_rsrc(args.lhs + bz * args.lhs_stride, args.lhs_bytes);
     const __amdgpu_buffer_rsrc_t rr = make_rsrc(args.rhs + bz * args.rhs_stride, args.rhs_bytes);
+    const __amdgpu_buffer_rsrc_t rc = make_rsrc(args.col_indices + start, (u32)(end - start) * 4u);
     int *const out = args.out + bz * args.out_stride;
 
     // K runs in passes of up to NKC 64-deep chunks; every pass holds its A
@@ -147,36 +171,73 @@ __global__ __launch_bounds__(64 * W) void sddmm_kernel(SddmmArgs args) {
     const int passes = (chunks + NKC - 1) / NKC;
     const bool a_live = r < ROWS;
     const int a_p = r / V, a_v = r % V;
+    const int perm_addr = 4 * (4 * r + g);
     for (int ps = 0; ps < passes; ++ps) {
         const int kc0 = ps * NKC;
         const int kn = min(NKC, chunks - kc0);   // chunks of this pass (uniform)
 
-        // A operands (lhs rows of this vector row) for the pass's chunks, and
-        // their digit row sums for the offset correction.
-        v4i aop[NKC];
-        int rsum = 0;
+        // column indices of a group's tiles (lane: slot 16 tile + lane / 4)
+        auto load_idx = [&](int tg, u32 (&idx)[TPW]) {
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) {
+                const int rel = (tg + t) * 16 + (lane >> 2);   // slot - start
+                idx[t] = buf_load_b32(rc, start + rel < end ? (u32)rel * 4u : 0x80000000u);
+            }
+        };
+        // raw gathered rows of a group; slots past the row end, negative
+        // indices and chunks past the pass read out of range (rhs < 1 GiB, so
+        // the offsets stay below 2^32 and outside the buffer)
+        auto gather = [&](int tg, const u32 (&idx)[TPW], v4i (&raw)[TPW][NKC][BD]) {
+#pragma unroll
+            for (int t = 0; t < TPW; ++t) {
+                // bitwise: one select, no branch around a wait
+                const bool in = (start + (tg + t) * 16 + (lane >> 2) < end) & ((int)idx[t] >= 0);
+                const u32 row = idx[t] * row_bytes;
+                const u32 o = (in ? row : kSddmmOob) + (u32)(16 * (lane & 3) * BITS / 8);
+#pragma unroll
+                for (int kc = 0; kc < NKC; ++kc) {
+                    const u32 ko = o + (kc < kn ? (u32)((kc0 + kc) * KB) : kSddmmOob);
+                    raw[t][kc][0] = load_k16<W16 ? 8 : BITS>(rr, ko);
+                    if constexpr (W16) raw[t][kc][1] = buf_load_b128(rr, ko + 16u);
+                }
+            }
+        };
+
+        constexpr int DEPTH = 2 * TPW * NKC * BD <= 16 ? 2 : 1;
+        u32 ia[TPW], ib[TPW];
+        v4i ra[TPW][NKC][BD], rb[DEPTH == 2 ? TPW : 1][NKC][BD];
+        load_idx(wave * TPW, ia);
+        load_idx(wave * TPW + step, ib);
+
+        // A operands (lhs rows of this vector row) for the pass's chunks
+        v4i aop[NKC], ahi[W16 ? NKC : 1];
 #pragma unroll
         for (int kc = 0; kc < NKC; ++kc) {
             const bool live = a_live && kc < kn;
             const u32 off =
                 live ? (u32)(m * V + a_v) * row_bytes + (u32)((kc0 + kc) * KB + 16 * g * BITS / 8) : 0x80000000u;
-            v4i x;
+            if constexpr (W16) load_k16_w16(rl, off, XHI, XLO, ahi[kc], aop[kc]);
+            else aop[kc] = load_k16<BITS>(rl, off);
+        }
+        gather(wave * TPW, ia, ra);
+        __builtin_amdgcn_sched_barrier(0);
+
+        // their digits, and the digit row sums for the offset correction
+        int rsum = 0;
+#pragma unroll
+        for (int kc = 0; kc < NKC; ++kc) {
+            v4i x = aop[kc];
             if constexpr (W16) {
-                v4i hi, lo;
-                load_k16_w16(rl, off, XHI, XLO, hi, lo);
                 // dead rows and chunks load nothing (offset out of range) but
                 // keep the XOR masks: zero them so they sum to 0
-                x = live ? (a_p == 0 ? hi : lo) : v4i{0, 0, 0, 0};
-            } else {
-                x = load_k16<BITS>(rl, off);
-            }
-            if constexpr (BITS == 8) {
+                x = a_live && kc < kn ? (a_p == 0 ? ahi[kc] : x) : v4i{0, 0, 0, 0};
+            } else if constexpr (BITS == 8) {
                 if constexpr (!SGN) {
                     const int sh = a_p == 0 ? 4 : 0;
 #pragma unroll
                     for (int q = 0; q < 4; ++q) x[q] = (int)(((u32)x[q] >> sh) & 0x0F0F0F0Fu);
                 }
-            } else if constexpr (BITS == 4) {
+            } else {
                 x = expand_nibbles(x, SGN, 0u);
             }
             aop[kc] = x;
@@ -197,165 +258,176 @@ __global__ __launch_bounds__(64 * W) void sddmm_kernel(SddmmArgs args) {
             }
         }
 
-        {
-            const int ctiles = (wend - start + 15) >> 4;
-            const __amdgpu_buffer_rsrc_t rc = make_rsrc(args.col_indices + start, (u32)(end - start) * 4u);
-            // wave w handles tile groups w, w + W, ... of TPW tiles each
-            for (int tg = wave * TPW; tg < ctiles; tg += W * TPW) {
-                constexpr int BD = W16 ? 2 : 1;   // rhs digits (16-bit: low, high)
-                v4i bop[TPW][NKC][BD];
-                int bsum[TPW];                    // sum of rhs' over this lane's k (16-bit)
-                // each wave loads the column indices of its own tiles (lane r:
-                // slot 16 tile + r) as rhs row byte offsets, out of range past
-                // the row end and for tiles past the row's last
-                u32 row_off[TPW];
+        // products of one tile, recombined and stored
+        auto consume = [&](int tile, const v4i (&raw)[NKC][BD]) {
+            v4i acc[BD];
 #pragma unroll
-                for (int t = 0; t < TPW; ++t) {
-                    const int rel = (tg + t) * 16 + r;   // slot - start
-                    const bool in = tg + t < ctiles && start + rel < end;
-                    const int idx = (int)buf_load_b32(rc, in ? (u32)rel * 4u : 0x80000000u);
-                    row_off[t] = in && idx >= 0 ? (u32)idx * row_bytes : kSddmmOob;
+            for (int q = 0; q < BD; ++q) acc[q] = v4i{0, 0, 0, 0};
+            int bsum = 0;                    // sum of rhs' over this lane's k (16-bit)
+#pragma unroll
+            for (int kc = 0; kc < NKC; ++kc) {
+                if constexpr (W16) {
+                    v4i hi, lo;
+                    split_w16(raw[kc][0], raw[kc][BD - 1], XHI, XLO, hi, lo);
+                    hi = row_to_operand(hi, perm_addr);
+                    lo = row_to_operand(lo, perm_addr);
+                    if (kc >= kn) { hi = v4i{0, 0, 0, 0}; lo = v4i{0, 0, 0, 0}; }
+                    bsum += 256 * sum_bytes(hi) + sum_bytes(lo);
+                    acc[0] = mfma_i8(aop[kc], lo, acc[0]);
+                    acc[BD - 1] = mfma_i8(aop[kc], hi, acc[BD - 1]);
+                } else {
+                    v4i x = row_to_operand<BITS == 4 ? 2 : 4>(raw[kc][0], perm_addr);
+                    if constexpr (BITS == 4) {
+                        x = expand_nibbles(x, false, SGN ? 0x88888888u : 0u);
+                    } else if constexpr (!SGN) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) x[q] = (int)((u32)x[q] ^ 0x80808080u);
+                    }
+                    acc[0] = mfma_i8(aop[kc], x, acc[0]);
                 }
+            }
+            // rhs digit sum of nonzero r over the pass's k (16-bit only)
+            u32 corr = 0;
+            if constexpr (W16) {
+                int sb = bsum;
+                sb += lane_read(sb, lane ^ 16);
+                sb += lane_read(sb, lane ^ 32);
+                corr = (u32)D::OA * (u32)sb + (u32)(64 * kn) * (u32)D::OA * (u32)OB;
+            }
+            // recombine digit planes into the home lanes (rows v = 4g + i),
+            // mod 2^32 in unsigned arithmetic
+            int res[HOME];
 #pragma unroll
-                for (int t = 0; t < TPW; ++t) {
-                    const u32 o = row_off[t];
-                    bsum[t] = 0;
+            for (int i = 0; i < HOME; ++i) {
+                u32 vsum = (u32)OB * (u32)rs_home[i] + corr;
 #pragma unroll
-                    for (int kc = 0; kc < NKC; ++kc) {
-                        // chunks past the pass read out of range (B < 1 GiB, so
-                        // o + kSddmmOob stays below 2^32 and outside the buffer)
-                        const u32 ko = o + (kc < kn ? (u32)((kc0 + kc) * KB) : kSddmmOob);
-                        if constexpr (W16) {
-                            v4i hi, lo;
-                            load_k16_w16(rr, ko + (u32)(32 * g), XHI, XLO, hi, lo);
-                            if (kc >= kn) { hi = v4i{0, 0, 0, 0}; lo = v4i{0, 0, 0, 0}; }
-                            bop[t][kc][0] = lo;
-                            bop[t][kc][BD - 1] = hi;
-                            bsum[t] += 256 * sum_bytes(hi) + sum_bytes(lo);
-                            continue;
-                        }
-                        v4i x = load_k16<BITS>(rr, ko + (u32)(16 * g * BITS / 8));
-                        if constexpr (BITS == 8) {
-                            if constexpr (!SGN) {
-#pragma unroll
-                                for (int q = 0; q < 4; ++q) x[q] = (int)((u32)x[q] ^ 0x80808080u);
-                            }
-                        } else {
-                            x = expand_nibbles(x, false, SGN ? 0x88888888u : 0u);
-                        }
-                        bop[t][kc][0] = x;
-                    }
+                for (int p = 0; p < P; ++p) {
+                    int dg, di;
+                    if constexpr (V == 8) { dg = 2 * (p % 2); di = 0; }
+                    else if constexpr (V == 4) { dg = p % 4; di = 0; }
+                    else { dg = (p % 8) / 2; di = 2 * (p % 2); }
+                    u32 x = (u32)acc[0][i + di];
+                    if constexpr (W16) x += (u32)acc[1][i + di] << 8;
+                    if (dg != 0) x = (u32)lane_down((int)x, 16 * dg);
+                    vsum += (u32)D::weight(p) * x;
                 }
+                res[i] = (int)vsum;
+            }
+            const int j = start + tile * 16 + r;
+            if constexpr (OUT == kOutHalf && V == 8) {
+                // lanes 32..63 take rows 2, 3 of each group of four, so that
+                // every lane divides two values instead of half of them four
+                const int two[2] = {
+                    (int)__builtin_amdgcn_permlane32_swap((u32)res[0], (u32)res[2], false, false)[0],
+                    (int)__builtin_amdgcn_permlane32_swap((u32)res[1], (u32)res[3], false, false)[0]};
+                const int row0 = 4 * (g & 1) + 2 * (g >> 1);
+                const float q[2] = {quotient_fast((float)two[0], args.div.d, args.div.y),
+                                    quotient_fast((float)two[1], args.div.d, args.div.y)};
+                const __half2 h = __floats2half2_rn(j < end ? q[0] : 0.f, j < end ? q[1] : 0.f);
+                if (j < wend)
+                    *reinterpret_cast<__half2 *>(args.out16 + bz * args.out_stride + (size_t)j * V + row0) = h;
+                return;
+            }
+            if constexpr (OUT == kOutHalf) {
+                if (g == 0 && j < wend) {
+                    float q[HOME];
 #pragma unroll
-                for (int t = 0; t < TPW; ++t) {
-                    v4i acc[BD];
+                    for (int i = 0; i < HOME; ++i) q[i] = quotient_fast((float)res[i], args.div.d, args.div.y);
+                    __half2 h[HOME / 2];
 #pragma unroll
-                    for (int q = 0; q < BD; ++q) {
-                        acc[q] = v4i{0, 0, 0, 0};
+                    for (int i = 0; i < HOME / 2; ++i)
+                        h[i] = __floats2half2_rn(j < end ? q[2 * i] : 0.f, j < end ? q[2 * i + 1] : 0.f);
+                    int *o = reinterpret_cast<int *>(args.out16 + bz * args.out_stride + (size_t)j * V);
+                    if constexpr (HOME == 4)
+                        *reinterpret_cast<v2i *>(o) =
+                            v2i{*reinterpret_cast<const int *>(&h[0]), *reinterpret_cast<const int *>(&h[1])};
+                    else
+                        *o = *reinterpret_cast<const int *>(&h[0]);
+                }
+                return;
+            }
+            // reference layout with four rows per lane: a 4 x 4 transpose
+            // within each quad of lanes gives lane r row 4g + (r & 3) of
+            // slots j4..j4+3 (j4 = j & ~3, start being a multiple of 8),
+            // one 16-byte run of [(j/8)][v][j%8].  A quad's four lanes are
+            // all in or all out of the store below (its slots share j4).
+            int tq[4] = {0, 0, 0, 0};
+            if constexpr (OUT_REF && HOME == 4) {
 #pragma unroll
-                        for (int kc = 0; kc < NKC; ++kc) acc[q] = mfma_i8(aop[kc], bop[t][kc][q], acc[q]);
-                    }
-                    // rhs digit sum of nonzero r over the pass's k (16-bit only)
-                    u32 corr = 0;
-                    if constexpr (W16) {
-                        int sb = bsum[t];
-                        sb += lane_read(sb, lane ^ 16);
-                        sb += lane_read(sb, lane ^ 32);
-                        corr = (u32)D::OA * (u32)sb + (u32)(64 * kn) * (u32)D::OA * (u32)OB;
-                    }
-                    // recombine digit planes into the home lanes (rows v = 4g + i),
-                    // mod 2^32 in unsigned arithmetic
-                    int res[HOME];
+                for (int i = 0; i < 4; ++i) tq[i] = j < end ? res[i] : 0;
+                quad_transpose4(tq, lane);
+            }
+            if (g < (V + 3) / 4 && j < wend) {
+                auto store_each = [&]() {
 #pragma unroll
                     for (int i = 0; i < HOME; ++i) {
-                        u32 vsum = (u32)OB * (u32)rs_home[i] + corr;
+                        const int v = 4 * g + i;
+                        const int val = j < end ? res[i] : 0;
+                        const size_t o = OUT_REF ? (size_t)(j >> 3) * 8 * V + 8 * v + (j & 7) : (size_t)j * V + v;
+                        // later passes add to what this lane stored before
+                        out[o] = ps == 0 ? val : (int)((u32)out[o] + (u32)val);
+                    }
+                };
+                if constexpr (HOME == 4) {
+                    if ((reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
+                        // [slot][V]: the lane's rows 4g..4g+3 are one 16-byte run
+                        const int j4 = j & ~3;
+                        const int v = 4 * g + (r & 3);
+                        v4i val = OUT_REF ? v4i{tq[0], tq[1], tq[2], tq[3]}
+                                          : (j < end ? v4i{res[0], res[1], res[2], res[3]} : v4i{0, 0, 0, 0});
+                        v4i *o = reinterpret_cast<v4i *>(
+                            out + (OUT_REF ? (size_t)(j4 >> 3) * 8 * V + 8 * v + (j4 & 7) : (size_t)j * V + 4 * g));
+                        if (ps != 0) {
+                            const v4i prev = *o;
 #pragma unroll
-                        for (int p = 0; p < P; ++p) {
-                            int dg, di;
-                            if constexpr (V == 8) { dg = 2 * (p % 2); di = 0; }
-                            else if constexpr (V == 4) { dg = p % 4; di = 0; }
-                            else { dg = (p % 8) / 2; di = 2 * (p % 2); }
-                            u32 x = (u32)acc[0][i + di];
-                            if constexpr (W16) x += (u32)acc[1][i + di] << 8;
-                            if (dg != 0) x = (u32)lane_down((int)x, 16 * dg);
-                            vsum += (u32)D::weight(p) * x;
+                            for (int i = 0; i < 4; ++i) val[i] = (int)((u32)prev[i] + (u32)val[i]);
                         }
-                        res[i] = (int)vsum;
+                        *o = val;
+                    } else {
+                        store_each();
                     }
-                    const int j = start + (tg + t) * 16 + r;
-                    // reference layout with four rows per lane: a 4 x 4 transpose
-                    // within each quad of lanes gives lane r row 4g + (r & 3) of
-                    // slots j4..j4+3 (j4 = j & ~3, start being a multiple of 8),
-                    // one 16-byte run of [(j/8)][v][j%8].  A quad's four lanes are
-                    // all in or all out of the store below (its slots share j4).
-                    int tq[4] = {0, 0, 0, 0};
-                    if constexpr (OUT_REF && HOME == 4) {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) tq[i] = j < end ? res[i] : 0;
-                        quad_transpose4(tq, lane);
-                    }
-                    if constexpr (OUT == kOutHalf) {
-                        if (g < (V + 3) / 4 && tg + t < ctiles && j < wend) {
-                            float q[HOME];
-                            int a[HOME];
-#pragma unroll
-                            for (int i = 0; i < HOME; ++i) a[i] = j < end ? res[i] : 0;
-                            divide<HOME>(a, args.div, q);
-                            __half2 h[HOME / 2];
-#pragma unroll
-                            for (int i = 0; i < HOME / 2; ++i) h[i] = __floats2half2_rn(j < end ? q[2 * i] : 0.f, j < end ? q[2 * i + 1] : 0.f);
-                            int *o = reinterpret_cast<int *>(args.out16 + bz * args.out_stride + (size_t)j * V + 4 * g);
-                            if constexpr (HOME == 4) *reinterpret_cast<v2i *>(o) = v2i{*reinterpret_cast<const int *>(&h[0]), *reinterpret_cast<const int *>(&h[1])};
-                            else *o = *reinterpret_cast<const int *>(&h[0]);
-                        }
-                        continue;
-                    }
-                    if (g < (V + 3) / 4 && tg + t < ctiles && j < wend) {
-                        auto store_each = [&]() {
-#pragma unroll
-                            for (int i = 0; i < HOME; ++i) {
-                                const int v = 4 * g + i;
-                                const int val = j < end ? res[i] : 0;
-                                const size_t o =
-                                    OUT_REF ? (size_t)(j >> 3) * 8 * V + 8 * v + (j & 7) : (size_t)j * V + v;
-                                // later passes add to what this lane stored before
-                                out[o] = ps == 0 ? val : (int)((u32)out[o] + (u32)val);
-                            }
-                        };
-                        if constexpr (OUT_REF && HOME == 4) {
-                            if ((reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
-                                const int j4 = j & ~3;
-                                const int v = 4 * g + (r & 3);
-                                v4i val = v4i{tq[0], tq[1], tq[2], tq[3]};
-                                v4i *o = reinterpret_cast<v4i *>(out + (size_t)(j4 >> 3) * 8 * V + 8 * v + (j4 & 7));
-                                if (ps != 0) {
-                                    const v4i prev = *o;
-#pragma unroll
-                                    for (int i = 0; i < 4; ++i) val[i] = (int)((u32)prev[i] + (u32)val[i]);
-                                }
-                                *o = val;
-                            } else {
-                                store_each();
-                            }
-                        } else if constexpr (!OUT_REF && HOME == 4) {
-                            if ((reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
-                                // [slot][V]: the lane's rows 4g..4g+3 are one 16-byte run
-                                v4i val = j < end ? v4i{res[0], res[1], res[2], res[3]} : v4i{0, 0, 0, 0};
-                                v4i *o = reinterpret_cast<v4i *>(out + (size_t)j * V + 4 * g);
-                                if (ps != 0) {
-                                    const v4i prev = *o;
-#pragma unroll
-                                    for (int i = 0; i < 4; ++i) val[i] = (int)((u32)prev[i] + (u32)val[i]);
-                                }
-                                *o = val;
-                            } else {
-                                store_each();
-                            }
-                        } else {
-                            store_each();
-                        }
-                    }
+                } else {
+                    store_each();
                 }
+            }
+        };
+
+        // a group's products; its last tiles may lie past the row (uniform)
+        auto consume_group = [&](int tg, const v4i (&raw)[TPW][NKC][BD]) {
+#pragma unroll
+            for (int t = 0; t < TPW; ++t)
+                if (tg + t < ctiles) consume(tg + t, raw[t]);
+        };
+        int tg = wave * TPW;
+        if (tg >= ctiles) continue;
+        if constexpr (DEPTH == 2) {
+            // the last group is written out of the loop, so that nothing is
+            // loaded past the row and every wait count in the loop is exact
+            for (;;) {
+                if (tg + step >= ctiles) { consume_group(tg, ra); break; }
+                gather(tg + step, ib, rb);
+                load_idx(tg + 2 * step, ia);
+                __builtin_amdgcn_sched_barrier(0);
+                consume_group(tg, ra);
+                __builtin_amdgcn_sched_barrier(0);
+                tg += step;
+                if (tg + step >= ctiles) { consume_group(tg, rb); break; }
+                gather(tg + step, ia, ra);
+                load_idx(tg + 2 * step, ib);
+                __builtin_amdgcn_sched_barrier(0);
+                consume_group(tg, rb);
+                __builtin_amdgcn_sched_barrier(0);
+                tg += step;
+            }
+        } else {
+            // one set of gathered rows fits: the next gathers go out between a
+            // group's products and the group after it
+            for (;; tg += step) {
+                consume_group(tg, ra);
+                if (tg + step >= ctiles) break;
+                gather(tg + step, ib, ra);
+                load_idx(tg + 2 * step, ib);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     }

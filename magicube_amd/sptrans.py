@@ -129,7 +129,8 @@ def _bsddmm(bits, row_indices, row_offsets, column_indices, lhs_matrix, rhs_matr
         out = torch.empty((batch, nnz * vec_length) if batched else (nnz * vec_length,), dtype=torch.float16,
                           device=lhs.device)
         lib, st = _lib.lib(), _stream_handle(stream)
-        if k <= 512 and m_vec:        # K in one pass: the kernel stores fp16 itself
+        # K in one pass and a divisor the kernel's quotient covers: it stores fp16 itself
+        if k <= 512 and m_vec and 2.0 ** -60 <= abs(scale) <= 2.0 ** 60:
             _lib.check(lib.mc_sddmm_batched_f16(bits, batch, m_vec, k, n, _ptr(ri), _ptr(ro), _ptr(ci), nnz,
                                                 _ptr(lhs), m * k_int32 * 4, _ptr(rhs), n * k_int32 * 4, float(scale),
                                                 _ptr(out), nnz * vec_length, vec_length, st), f"bsddmm_{bits}b")
