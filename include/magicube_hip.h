@@ -267,6 +267,9 @@ typedef struct mc_quant_job {
  * device array of njobs jobs; max_count bounds every job's count. */
 mc_status mc_attn_quantize_batched(const mc_quant_job *jobs, int njobs, int bits, int rounding,
                                    long long max_count, hipStream_t stream);
+/* The same for one contiguous tensor, described by the arguments. */
+mc_status mc_attn_quantize(const void *x_fp16, long long count, float scale, int bits, int rounding, void *out,
+                           hipStream_t stream);
 /* max |x| of an fp16 tensor, as float bits combined into *out_bits (device,
  * zero-initialised by the caller) with atomicMax.  No reference counterpart
  * (the reference uses a fixed scale, spattention.py:51). */
@@ -306,6 +309,13 @@ mc_status mc_attn_softmax_f16(int batch, int rows, int vec_length, const int *ro
                               const int *row_offsets, const void *values_f16, long long values_stride,
                               float sqrt_dk, float scale, int bits, void *attn, long long attn_stride_bytes,
                               hipStream_t stream);
+
+/* Zeroes the slots of [0, slots) that no row writes: those outside every
+ * row's [start, start + roundup(nonzeros, group)), at slot_bits bits a slot
+ * (a multiple of 8), in each of `batch` outputs stride_bytes apart.  Rows may
+ * lie in any order; launched before the op that writes them. */
+mc_status mc_attn_zero_gaps(int batch, int rows, const int *row_offsets, int slots, int group, int slot_bits,
+                            void *out, long long stride_bytes, hipStream_t stream);
 
 /* One attention matrix of the fused batched launch (device-resident
  * descriptor).  q, k: [L][64] int8 (or int4 packed [L][32] bytes); v: [L][64]

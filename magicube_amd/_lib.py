@@ -48,6 +48,7 @@ _SIGS["mc_sddmm_run"] = (_I, [_I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _I
 _F = ctypes.c_float
 _LL = ctypes.c_longlong
 _SIGS["mc_attn_quantize_batched"] = (_I, [_P, _I, _I, _I, _LL, _P])
+_SIGS["mc_attn_quantize"] = (_I, [_P, _LL, _F, _I, _I, _P, _P])
 _SIGS["mc_attn_absmax"] = (_I, [_P, _LL, _P, _P])
 _SIGS["mc_attn_softmax_requant"] = (_I, [_I, _I, _P, _P, _P, _F, _F, _I, _P, _P, _P])
 _SIGS["mc_attn_dequant"] = (_I, [_P, _I, _I, _F, _P, _P, _P])
@@ -55,6 +56,7 @@ _SIGS["mc_attn_forward"] = (_I, [_P, _P, _I, _I, _I, _I, _F, _I, _I, _I, _P])
 _SIGS["mc_attn_dequant_f16"] = (_I, [_P, _LL, _F, _P, _P])
 _SIGS["mc_layernorm_f16"] = (_I, [_LL, _I, _P, _P, _P, _P, _F, _P, _P])
 _SIGS["mc_attn_softmax_f16"] = (_I, [_I, _I, _I, _P, _P, _P, _LL, _F, _F, _I, _P, _LL, _P])
+_SIGS["mc_attn_zero_gaps"] = (_I, [_I, _I, _P, _I, _I, _I, _P, _LL, _P])
 _SIGS["mc_spmm_batched"] = (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _LL, _P, _LL, _P, _LL, _P])
 _SIGS["mc_spmm_batched_f16"] = (_I, [_I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _LL, _P, _LL, _F, _P, _LL, _P])
 _SIGS["mc_sddmm_batched_f16"] = (_I, [_I, _I, _I, _I, _I, _P, _P, _P, _I, _P, _LL, _P, _LL, _F, _P, _LL, _I, _P])

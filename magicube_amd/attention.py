@@ -711,8 +711,8 @@ def bquantization(x: torch.Tensor, bits: int, scale: float, rounding: int = ROUN
     D * bits must be a multiple of 32 (the reference passes D = 64).
 
     Runs on ``stream`` (default: the current stream), which must see ``x``
-    ready.  The contiguous copy of ``x``, the job descriptor and the output
-    are made on that stream too, so the caching allocator cannot hand their
+    ready.  The contiguous copy of ``x`` and the output are made on that
+    stream too, so the caching allocator cannot hand their
     memory to other work before the launch has read or written it."""
     if bits not in (8, 4):
         raise ValueError("bits must be 8 or 4")
@@ -724,9 +724,8 @@ def bquantization(x: torch.Tensor, bits: int, scale: float, rounding: int = ROUN
     with ctx:
         x = x.contiguous()
         out = torch.empty(x.shape[:-1] + (x.shape[-1] * bits // 32,), dtype=torch.int32, device=x.device)
-        job = _struct_tensor([_QuantJobC(x.data_ptr(), x.numel(), float(scale), out.data_ptr())], x.device)
-        _lib.check(_lib.lib().mc_attn_quantize_batched(_dptr(job), 1, bits, rounding, x.numel(), _stream(stream)),
-                   "bquantization")
+        _lib.check(_lib.lib().mc_attn_quantize(_dptr(x), x.numel(), float(scale), bits, rounding, _dptr(out),
+                                               _stream(stream)), "bquantization")
     return out
 
 

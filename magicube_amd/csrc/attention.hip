@@ -3,6 +3,8 @@
 // work item, persistent over a longest-first work list), plus the C ABI.
 #include <hip/hip_fp16.h>
 
+#include <type_traits>
+
 #include "attention_common.hpp"
 #include "mc_internal.hpp"
 #include "sddmm_kernel.hpp"
@@ -52,42 +54,73 @@ static_assert(sizeof(QuantJob) == sizeof(mc_quant_job), "job layout");
 
 // Groups of 8 consecutive values that one thread converts per pass: the
 // block covers 256 * kQuantGroups groups, thread t takes groups t, t + 256,
-// ... of them, and all of its loads are issued before any is converted
-// (two 16-byte loads in flight per thread; one or four measured slower).
+// ... of them, and all of its loads are issued before any is converted.
 constexpr int kQuantGroups = 2;
 
+// the job's pointers come from memory: without the address space every access
+// is a flat one, whose loads also wait for LDS
+typedef __attribute__((address_space(1))) const v4i global_v4i;
+typedef __attribute__((address_space(1))) v2i global_v2i;
+typedef __attribute__((address_space(1))) u32 global_u32;
+
+// 8 values -> 8 int8 or packed int4 at group gi of the job's output
 template <int BITS>
-__global__ __launch_bounds__(256) void quantize_kernel(const QuantJob *jobs, int njobs, int rounding) {
-    const QuantJob jb = jobs[blockIdx.y];
+__device__ __forceinline__ void quantize_group(const float (&x)[8], const QuantJob &jb, int rounding, float lo,
+                                               float hi, long long gi) {
+    int q[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        float f = x[e] * jb.scale;
+        f = fminf(fmaxf(f, lo), hi);
+        q[e] = (rounding & 1) == 0 ? (int)f : (int)rintf(f);
+    }
+    if constexpr (BITS == 8) {
+        unsigned char *o = static_cast<unsigned char *>(jb.out) + gi * 8;
+        if (gi * 8 + 8 <= jb.count) {
+            u32 w0 = (u32)(q[0] & 255) | (u32)(q[1] & 255) << 8 | (u32)(q[2] & 255) << 16 | (u32)(q[3] & 255) << 24;
+            u32 w1 = (u32)(q[4] & 255) | (u32)(q[5] & 255) << 8 | (u32)(q[6] & 255) << 16 | (u32)(q[7] & 255) << 24;
+            *(global_v2i *)o = v2i{(int)w0, (int)w1};
+        } else {
+            for (int e = 0; gi * 8 + e < jb.count; ++e) o[e] = (unsigned char)q[e];
+        }
+    } else {
+        u32 wq = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) wq |= (u32)(q[e] & 15) << (4 * e);
+        *((global_u32 *)jb.out + gi) = wq;
+    }
+}
+
+template <int BITS> __device__ __forceinline__ void quantize_job(const QuantJob jb, int rounding) {
     // MC_QUANT_RANGE4 (bit 1 of rounding): 4-bit values in int8 storage
     const bool range4 = BITS == 4 || (rounding & 2) != 0;
     const float lo = range4 ? -8.f : -128.f, hi = range4 ? 7.f : 127.f;
     constexpr int G = kQuantGroups;
     const long long groups = (jb.count + 7) / 8;
-    for (long long blk = blockIdx.x; blk * 256 * G < groups; blk += gridDim.x) {
-        const long long g0 = blk * 256 * G + threadIdx.x;
-        v4i w[G];
-        bool fast[G];
+    // Whole groups of a job whose rows start on 16 bytes and are 2^shift long
+    // (every head dimension; shift 62: contiguous) take the branch-free loop:
+    // clamped 16-byte loads, so that a thread's loads are in flight together.
+    // Non-temporal: the fp16 source is read once, and keeping it out of the
+    // caches leaves them to the quantized operands the fused kernel gathers
+    // next.
+    const bool regular = (jb.row_len & (jb.row_len - 1)) == 0 &&
+                         (reinterpret_cast<uintptr_t>(jb.x) & 15u) == 0 && (jb.row_len == 0 || jb.row_stride % 8 == 0);
+    long long done = 0;     // groups the first loop converts
+    if (regular && jb.count >= 8) {
+        const int shift = jb.row_len == 0 ? 62 : (int)__ffsll((unsigned long long)jb.row_len) - 1;
+        const long long skip = jb.row_len == 0 ? 0 : jb.row_stride - jb.row_len;
+        done = jb.count / 8;
+        for (long long blk = blockIdx.x; blk * 256 * G < done; blk += gridDim.x) {
+            const long long g0 = blk * 256 * G + threadIdx.x;
+            v4i w[G];
 #pragma unroll
-        for (int k = 0; k < G; ++k) {
-            const long long gi = g0 + 256 * k;
-            const long long base = gi * 8;
-            // the 8 values never straddle a source row (row_len % 8 == 0)
-            const __half *src = jb.row_len ? jb.x + (base / jb.row_len) * jb.row_stride + base % jb.row_len
-                                           : jb.x + base;
-            fast[k] = gi < groups && base + 8 <= jb.count && (reinterpret_cast<uintptr_t>(src) & 15u) == 0;
-            // one 16-byte load for the 8 values, non-temporal: the fp16 source is
-            // read once, and keeping it out of the caches leaves them to the
-            // quantized operands the fused kernel gathers next
-            if (fast[k]) w[k] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(src));
-        }
+            for (int k = 0; k < G; ++k) {
+                const long long base = min(g0 + 256 * k, done - 1) * 8;
+                w[k] = __builtin_nontemporal_load((global_v4i *)(jb.x + base + (base >> shift) * skip));
+            }
 #pragma unroll
-        for (int k = 0; k < G; ++k) {
-            const long long gi = g0 + 256 * k;
-            if (gi >= groups) continue;
-            const long long base = gi * 8;
-            float x[8];
-            if (fast[k]) {
+            for (int k = 0; k < G; ++k) {
+                float x[8];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int we = w[k][e];
@@ -95,37 +128,31 @@ __global__ __launch_bounds__(256) void quantize_kernel(const QuantJob *jobs, int
                     x[2 * e] = __low2float(h2);
                     x[2 * e + 1] = __high2float(h2);
                 }
-            } else {
-                const __half *src = jb.row_len ? jb.x + (base / jb.row_len) * jb.row_stride + base % jb.row_len
-                                               : jb.x + base;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) x[e] = base + e < jb.count ? __half2float(src[e]) : 0.f;
-            }
-            int q[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                float f = x[e] * jb.scale;
-                f = fminf(fmaxf(f, lo), hi);
-                q[e] = (rounding & 1) == 0 ? (int)f : (int)rintf(f);
-            }
-            if constexpr (BITS == 8) {
-                unsigned char *o = static_cast<unsigned char *>(jb.out) + base;
-                if (base + 8 <= jb.count) {
-                    u32 w0 = (u32)(q[0] & 255) | (u32)(q[1] & 255) << 8 | (u32)(q[2] & 255) << 16 | (u32)(q[3] & 255) << 24;
-                    u32 w1 = (u32)(q[4] & 255) | (u32)(q[5] & 255) << 8 | (u32)(q[6] & 255) << 16 | (u32)(q[7] & 255) << 24;
-                    *reinterpret_cast<v2i *>(o) = v2i{(int)w0, (int)w1};
-                } else {
-                    for (int e = 0; base + e < jb.count; ++e) o[e] = (unsigned char)q[e];
-                }
-            } else {
-                u32 wq = 0;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) wq |= (u32)(q[e] & 15) << (4 * e);
-                static_cast<u32 *>(jb.out)[gi] = wq;
+                if (g0 + 256 * k < done) quantize_group<BITS>(x, jb, rounding, lo, hi, g0 + 256 * k);
             }
         }
     }
-    (void)njobs;
+    // the rest value by value: the last part of a group, unaligned or
+    // irregular rows (8 values never straddle a source row: row_len % 8 == 0)
+    for (long long gi = done + (long long)blockIdx.x * 256 + threadIdx.x; gi < groups; gi += (long long)gridDim.x * 256) {
+        const long long base = gi * 8;
+        const __half *src = jb.row_len ? jb.x + (base / jb.row_len) * jb.row_stride + base % jb.row_len : jb.x + base;
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = base + e < jb.count ? __half2float(src[e]) : 0.f;
+        quantize_group<BITS>(x, jb, rounding, lo, hi, gi);
+    }
+}
+
+// One job per blockIdx.y from a device array, or the one job passed as an
+// argument (a single tensor: no descriptor to copy to the device first).
+template <int BITS>
+__global__ __launch_bounds__(256) void quantize_kernel(const QuantJob *jobs, int rounding) {
+    const QuantJob job = jobs[blockIdx.y];       // a copy: stores to its output cannot change it
+    quantize_job<BITS>(job, rounding);
+}
+template <int BITS> __global__ __launch_bounds__(256) void quantize_one_kernel(QuantJob job, int rounding) {
+    quantize_job<BITS>(job, rounding);
 }
 
 // max |x| over a tensor, combined with atomicMax on the float bit pattern
@@ -253,105 +280,222 @@ __global__ __launch_bounds__(256) void dequant_f16_kernel(const int *in, long lo
 // 4-bit P, else 16), padding slots with 0.  The sum runs in a fixed order:
 // lane l adds slots l, l + 64, ..., then a butterfly over the 64 lanes.
 // ---------------------------------------------------------------------------
-template <int V>
-__device__ __forceinline__ void load_half_vec(const __half *p, float (&x)[V]) {
-    if constexpr (V == 8) {
-        const v4i w = *reinterpret_cast<const v4i *>(p);
+// A slot's V fp16 logits, packed two to a register.
+template <int V> struct HalfVec {
+    u32 w[V / 2];
+    __device__ __forceinline__ float at(int v) const {
+        const __half2 h2 = *reinterpret_cast<const __half2 *>(&w[v >> 1]);
+        return v & 1 ? __high2float(h2) : __low2float(h2);
+    }
+    // element-wise maximum (of a NaN and a number, the number)
+    __device__ __forceinline__ void take_max(const HalfVec &o) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int we = w[e];
-            const __half2 h2 = *reinterpret_cast<const __half2 *>(&we);
-            x[2 * e] = __low2float(h2);
-            x[2 * e + 1] = __high2float(h2);
+        for (int k = 0; k < V / 2; ++k) {
+            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+            const h2 r = __builtin_elementwise_max(*reinterpret_cast<const h2 *>(&w[k]),
+                                                   *reinterpret_cast<const h2 *>(&o.w[k]));
+            w[k] = *reinterpret_cast<const u32 *>(&r);
         }
+    }
+};
+template <int V> __device__ __forceinline__ HalfVec<V> load_half_vec(const __half *p) {
+    HalfVec<V> x;
+    if constexpr (V == 8) {
+        const v4i t = *reinterpret_cast<const v4i *>(p);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x.w[e] = (u32)t[e];
     } else {
 #pragma unroll
-        for (int v = 0; v < V; ++v) x[v] = __half2float(p[v]);
+        for (int k = 0; k < V / 2; ++k) {
+            const __half2 t{p[2 * k], p[2 * k + 1]};
+            x.w[k] = *reinterpret_cast<const u32 *>(&t);
+        }
     }
+    return x;
 }
 
+// Butterflies over the wave without LDS: within each row of 16 lanes by DPP
+// (row16_max / row16_sum), then v_permlane16_swap and v_permlane32_swap give
+// every lane its own and its partner row's value.  The sum adds the same
+// pairs as the xor butterfly over lane distances 1, 2, 4, 8, 16, 32.
 __device__ __forceinline__ float wave_max(float x) {
-    for (int s = 32; s > 0; s >>= 1) x = fmaxf(x, __shfl_xor(x, s, 64));
-    return x;
+    x = row16_max(x);
+    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
 }
 __device__ __forceinline__ float wave_sum(float x) {
-    for (int s = 1; s < 64; s <<= 1) x += __shfl_xor(x, s, 64);
-    return x;
+    x = row16_sum(x);
+    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(a[0]) + __uint_as_float(a[1]);
 }
 
+// 4 x 4 byte transpose within each quad of lanes: lane q gets byte q of its
+// quad's four dwords (lane k's as byte k).
+__device__ __forceinline__ u32 quad_bytes(u32 x, u32 sel) {
+    const u32 d0 = (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x00, 0xF, 0xF, false);
+    const u32 d1 = (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0x55, 0xF, 0xF, false);
+    const u32 d2 = (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0xAA, 0xF, 0xF, false);
+    const u32 d3 = (u32)__builtin_amdgcn_update_dpp(0, (int)x, 0xFF, 0xF, 0xF, false);
+    return perm(perm(d3, d2, sel), perm(d1, d0, sel), 0x05040100u);
+}
+
+// One wave per (vector row, matrix); lane l holds slots l, l + 64, ...  Bound
+// by its instructions (13 million logits, three passes), so: the logits of a
+// row's first NC chunks are read once and their exponentials kept in
+// registers (rows beyond that are read again), the division by the row sum
+// is a host-free corrected reciprocal (quotient_fast: the IEEE quotient)
+// while the sum and scale lie within 2^40 of 1, wave reductions use no LDS,
+// and each quad of lanes transposes its four slots' bytes, so that a row's
+// four slots go out as one dword instead of four bytes.
 template <int V, int BITS, int WPB>
 __global__ __launch_bounds__(64 * WPB) void ref_softmax_kernel(int rows, const int *row_indices, const int *row_offsets,
                                                                const __half *values, long long values_stride,
                                                                float sqrt_dk, float scale, unsigned char *attn,
                                                                long long attn_stride) {
+    constexpr int NC = V == 8 ? 8 : 16;          // chunks of 64 slots held in registers
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x = blockIdx.x * WPB + wave;
     if (x >= rows) return;
     const long long b = blockIdx.y;
     const int m = uniform(row_indices ? row_indices[x] : x);
     const int start = uniform(row_offsets[2 * m]), nz = uniform(row_offsets[2 * m + 1]) - start;
+    if (nz <= 0) return;                         // no slot to write
     const __half *val = values + b * values_stride + (size_t)start * V;
     unsigned char *out = attn + b * attn_stride + (size_t)start * V * BITS / 8;
 
+    HalfVec<V> h[NC];                            // logits
+    float s[NC][V];                              // their exponentials
     float mx[V], sm[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) { mx[v] = v == 0 ? -1e10f : 0.f; sm[v] = 0.f; }
-    for (int i = lane; i < nz; i += 64) {
-        float s[V];
-        load_half_vec<V>(val + (size_t)i * V, s);
+    // lanes past the end repeat the last slot: it changes no maximum
 #pragma unroll
-        for (int v = 0; v < V; ++v) mx[v] = fmaxf(mx[v], s[v] * sqrt_dk);
+    for (int c = 0; c < NC; ++c)
+        if (64 * c < nz) h[c] = load_half_vec<V>(val + (size_t)min(64 * c + lane, nz - 1) * V);
+    const auto scaled_max = [&](const HalfVec<V> &t) {
+#pragma unroll
+        for (int v = 0; v < V; ++v) mx[v] = fmaxf(mx[v], t.at(v) * sqrt_dk);
+    };
+    // the maximum over logits first, scaled once: rounding keeps order, so
+    // for a positive factor it is the maximum of the scaled logits
+    if (sqrt_dk > 0.f) {
+        HalfVec<V> hm = h[0];
+#pragma unroll
+        for (int c = 1; c < NC; ++c)
+            if (64 * c < nz) hm.take_max(h[c]);
+        scaled_max(hm);
+    } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            if (64 * c < nz) scaled_max(h[c]);
     }
+    for (int i = 64 * NC + lane; i < nz; i += 64) scaled_max(load_half_vec<V>(val + (size_t)i * V));
 #pragma unroll
     for (int v = 0; v < V; ++v) mx[v] = wave_max(mx[v]);
-    for (int i = lane; i < nz; i += 64) {
-        float s[V];
-        load_half_vec<V>(val + (size_t)i * V, s);
+    const auto expo = [&](float t, int v) { return __expf(__builtin_fmaf(t, sqrt_dk, -mx[v])); };
 #pragma unroll
-        for (int v = 0; v < V; ++v) sm[v] += __expf(s[v] * sqrt_dk - mx[v]);
+    for (int c = 0; c < NC; ++c)
+        if (64 * c < nz) {
+#pragma unroll
+            for (int v = 0; v < V; ++v) s[c][v] = expo(h[c].at(v), v);
+            if (64 * c + 64 > nz) {
+                const bool in = 64 * c + lane < nz;
+#pragma unroll
+                for (int v = 0; v < V; ++v) s[c][v] = in ? s[c][v] : 0.f;
+            }
+#pragma unroll
+            for (int v = 0; v < V; ++v) sm[v] += s[c][v];
+        }
+    for (int i = 64 * NC + lane; i < nz; i += 64) {
+        const HalfVec<V> t = load_half_vec<V>(val + (size_t)i * V);
+#pragma unroll
+        for (int v = 0; v < V; ++v) sm[v] += expo(t.at(v), v);
     }
+    // fast: every quotient this row can give an integer from stays in the
+    // corrected reciprocal's range (an exponential below 2^-100 gives 0 with
+    // either division), and 0 <= exponential / sum * scale <= hi needs no
+    // clamp.  The sums are the same in every lane.
+    constexpr float lo = BITS == 4 ? -8.f : BITS == 8 ? -128.f : -32768.f;
+    constexpr float hi = BITS == 4 ? 7.f : BITS == 8 ? 127.f : 32767.f;
+    float y[V];
+    bool fast = scale >= 0.f && scale <= hi;
 #pragma unroll
-    for (int v = 0; v < V; ++v) sm[v] = wave_sum(sm[v]);
+    for (int v = 0; v < V; ++v) {
+        sm[v] = wave_sum(sm[v]);
+        y[v] = 1.0f / sm[v];
+        fast &= sm[v] >= 0x1p-40f && sm[v] <= 0x1p40f;
+    }
+    fast = __builtin_amdgcn_readfirstlane(fast) != 0;
 
-    auto prob = [&](int i, int v, const float (&s)[V], float lo, float hi) {
-        if (i >= nz) return 0.f;
-        const float p = __expf(s[v] * sqrt_dk - mx[v]) / sm[v] * scale;
-        return fminf(fmaxf(p, lo), hi);
+    const int q = lane & 3;
+    const u32 sel = (u32)q | (u32)(4 + q) << 8 | 0x0C0C0000u;
+    const bool aligned = (reinterpret_cast<uintptr_t>(out) & 3) == 0;
+    const auto store4 = [&](unsigned char *o, u32 w) {
+        if (aligned) *reinterpret_cast<u32 *>(o) = w;
+        else
+            for (int k = 0; k < 4; ++k) o[k] = (unsigned char)(w >> (8 * k));
     };
-    if constexpr (BITS == 4) {
-        // slot pairs (2j, 2j + 1) of 32-slot groups
-        const int npair = ((nz + 31) & ~31) / 2;
-        for (int j = lane; j < npair; j += 64) {
-            const int i = 2 * j;
-            float s0[V], s1[V];
-            if (i < nz) load_half_vec<V>(val + (size_t)i * V, s0);
-            if (i + 1 < nz) load_half_vec<V>(val + (size_t)(i + 1) * V, s1);
+    // P of the lane's slot 64c + lane from its exponentials; every slot of a
+    // quad is written or none (rows are padded to 16 or 32 slots with 0)
+    const int nw = BITS == 4 ? (nz + 31) & ~31 : (nz + 15) & ~15;
+    const auto write = [&](auto quick, int c, const float (&e)[V]) {
+        const int i = 64 * c + lane;
+        u32 p[V < 4 ? 4 : V];
+        if constexpr (V < 4) p[2] = p[3] = 0;
 #pragma unroll
-            for (int v = 0; v < V; ++v) {
-                const int p0 = (int)(signed char)prob(i, v, s0, -8.f, 7.f);
-                const int p1 = (int)(signed char)prob(i + 1, v, s1, -8.f, 7.f);
-                out[(size_t)(i >> 5) * V * 16 + 16 * v + (j & 15)] = (unsigned char)((p0 & 15) | (p1 << 4));
+        for (int v = 0; v < V; ++v) {
+            if constexpr (decltype(quick)::value) {
+                p[v] = (u32)(int)(quotient_fast(e[v], sm[v], y[v]) * scale);
+            } else {
+                const float cl = fminf(fmaxf(e[v] / sm[v] * scale, lo), hi);
+                p[v] = i < nz ? (u32)(int)cl : 0u;
             }
         }
-    } else {
-        const int nw = (nz + 15) & ~15;
-        for (int i = lane; i < nw; i += 64) {
-            float s[V];
-            if (i < nz) load_half_vec<V>(val + (size_t)i * V, s);
+        if (i >= nw) return;
 #pragma unroll
-            for (int v = 0; v < V; ++v) {
-                if constexpr (BITS == 8) {
-                    const int p = (int)(signed char)prob(i, v, s, -128.f, 127.f);
-                    out[(size_t)(i >> 4) * V * 16 + 16 * v + (i & 15)] = (unsigned char)p;
-                } else {
-                    const int p = (int)(short)prob(i, v, s, -32768.f, 32767.f);
-                    unsigned char *o = out + (size_t)(i >> 4) * V * 32 + 32 * v + (i & 15);
-                    o[0] = (unsigned char)(p & 255);
-                    o[16] = (unsigned char)((p >> 8) & 255);
+        for (int h = 0; h < V; h += 4) {
+            // rows h .. h + 3: lane q of the quad stores row h + q of its four slots
+            const int row = h + q;
+            const u32 w0 = (p[h] & 255) | (p[h + 1] & 255) << 8 | (p[h + 2] & 255) << 16 | p[h + 3] << 24;
+            if constexpr (BITS == 4) {
+                const u32 t = quad_bytes(w0 & 0x0F0F0F0Fu, sel);
+                const u32 y2 = t | t >> 4;
+                unsigned char *o = out + (size_t)(i >> 5) * V * 16 + 16 * row + ((i & 31) >> 2) * 2;
+                if (row < V) {
+                    if (aligned) *reinterpret_cast<unsigned short *>(o) = (unsigned short)perm(y2, y2, 0x0C0C0200u);
+                    else { o[0] = (unsigned char)y2; o[1] = (unsigned char)(y2 >> 16); }
+                }
+            } else {
+                unsigned char *o = out + (size_t)(i >> 4) * V * (2 * BITS) + 2 * BITS * row + ((i & 15) >> 2) * 4;
+                const u32 t = quad_bytes(w0, sel);
+                if (row < V) store4(o, t);
+                if constexpr (BITS == 16) {
+                    const u32 w1 = (p[h] >> 8 & 255) | (p[h + 1] >> 8 & 255) << 8 | (p[h + 2] >> 8 & 255) << 16 |
+                                   p[h + 3] >> 8 << 24;
+                    const u32 t1 = quad_bytes(w1, sel);
+                    if (row < V) store4(o + 16, t1);
                 }
             }
         }
-    }
+    };
+    const auto write_row = [&](auto quick) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            if (64 * c < nw) write(quick, c, s[c]);
+        for (int c = NC; 64 * c < nw; ++c) {
+            const HalfVec<V> t = load_half_vec<V>(val + (size_t)min(64 * c + lane, nz - 1) * V);
+            float e[V];
+#pragma unroll
+            for (int v = 0; v < V; ++v) e[v] = 64 * c + lane < nz ? expo(t.at(v), v) : 0.f;
+            write(quick, c, e);
+        }
+    };
+    if (fast) write_row(std::true_type{});
+    else write_row(std::false_type{});
 }
 
 // Row bounds are read-only for the whole launch; read through the constant
@@ -774,8 +918,23 @@ mc_status mc_attn_quantize_batched(const mc_quant_job *jobs, int njobs, int bits
     if (!jobs || njobs > 65535) return MC_EINVAL_ARG;
     const unsigned gx = grid_for((max_count + 7) / 8, 256 * mc::kQuantGroups);
     const auto *dj = reinterpret_cast<const mc::QuantJob *>(jobs);
-    if (bits == 8) hipLaunchKernelGGL(mc::quantize_kernel<8>, dim3(gx, njobs), dim3(256), 0, stream, dj, njobs, rounding);
-    else hipLaunchKernelGGL(mc::quantize_kernel<4>, dim3(gx, njobs), dim3(256), 0, stream, dj, njobs, rounding);
+    if (bits == 8) hipLaunchKernelGGL(mc::quantize_kernel<8>, dim3(gx, njobs), dim3(256), 0, stream, dj, rounding);
+    else hipLaunchKernelGGL(mc::quantize_kernel<4>, dim3(gx, njobs), dim3(256), 0, stream, dj, rounding);
+    return mc::check_launch();
+}
+
+mc_status mc_attn_quantize(const void *x_fp16, long long count, float scale, int bits, int rounding, void *out,
+                           hipStream_t stream) {
+    if (bits != 8 && bits != 4) return MC_EUNSUPPORTED;
+    if ((rounding & ~MC_QUANT_RANGE4) != MC_ROUND_TRUNC && (rounding & ~MC_QUANT_RANGE4) != MC_ROUND_NEAREST)
+        return MC_EINVAL_ARG;
+    if (count < 0) return MC_EINVAL_ARG;
+    if (count == 0) return MC_OK;
+    if (!x_fp16 || !out) return MC_EINVAL_ARG;
+    const unsigned gx = grid_for((count + 7) / 8, 256 * mc::kQuantGroups);
+    const mc::QuantJob job{static_cast<const __half *>(x_fp16), count, scale, out, 0, 0};
+    if (bits == 8) hipLaunchKernelGGL(mc::quantize_one_kernel<8>, dim3(gx), dim3(256), 0, stream, job, rounding);
+    else hipLaunchKernelGGL(mc::quantize_one_kernel<4>, dim3(gx), dim3(256), 0, stream, job, rounding);
     return mc::check_launch();
 }
 
@@ -838,6 +997,15 @@ mc_status mc_attn_softmax_f16(int batch, int rows, int vec_length, const int *ro
 #undef MC_REF_SOFTMAX_V
 #undef MC_REF_SOFTMAX
     return mc::check_launch();
+}
+
+mc_status mc_attn_zero_gaps(int batch, int rows, const int *row_offsets, int slots, int group, int slot_bits, void *out,
+                            long long stride_bytes, hipStream_t stream) {
+    if (batch < 1 || batch > 65535 || rows < 0 || slots < 0 || stride_bytes < 0) return MC_EINVAL_SHAPE;
+    if (group < 1 || slot_bits < 8 || slot_bits % 8 != 0) return MC_EINVAL_ARG;
+    if (slots == 0) return MC_OK;
+    if (!out || (rows > 0 && !row_offsets)) return MC_EINVAL_ARG;
+    return mc::zero_gaps(batch, rows, row_offsets, slots, group, slot_bits, out, stride_bytes, stream);
 }
 
 mc_status mc_attn_softmax_requant(int m_vec, int vec_length, const int *row_indices, const int *row_offsets,

@@ -195,10 +195,18 @@ def q_bcsr_softmax(row_indices, row_offsets, values, sqrt_dk: float, scale: floa
         raise ValueError(f"{stride} values per matrix do not pack into int32 words of {bits}-bit P")
     attn_stride = stride * bits // 32
     with _on(stream):
-        attn = torch.zeros((batch_size, attn_stride), dtype=torch.int32, device=vals.device)
-        _lib.check(_lib.lib().mc_attn_softmax_f16(batch_size, ri.numel(), vec_length, _ptr(ri), _ptr(ro), _ptr(vals),
-                                                  stride, float(sqrt_dk), float(scale), bits, _ptr(attn),
-                                                  attn_stride * 4, _stream_handle(stream)), "q_bcsr_softmax")
+        lib, st = _lib.lib(), _stream_handle(stream)
+        rows, slots = ri.numel(), stride // vec_length
+        if 2 * rows == ro.numel() and stride % vec_length == 0:
+            # every row is written: only the slots between rows need zeros
+            attn = torch.empty((batch_size, attn_stride), dtype=torch.int32, device=vals.device)
+            _lib.check(lib.mc_attn_zero_gaps(batch_size, rows, _ptr(ro), slots, 32 if bits == 4 else 16,
+                                             vec_length * bits, _ptr(attn), attn_stride * 4, st), "q_bcsr_softmax")
+        else:
+            attn = torch.zeros((batch_size, attn_stride), dtype=torch.int32, device=vals.device)
+        _lib.check(lib.mc_attn_softmax_f16(batch_size, rows, vec_length, _ptr(ri), _ptr(ro), _ptr(vals), stride,
+                                           float(sqrt_dk), float(scale), bits, _ptr(attn), attn_stride * 4, st),
+                   "q_bcsr_softmax")
     return attn
 
 

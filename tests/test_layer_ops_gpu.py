@@ -93,3 +93,53 @@ def test_bsddmm_edges(bits, k, V, layout):
     torch.cuda.synchronize()
     exp = oatt.ref_bsddmm(lhs, rhs, pairs, cols, V, divisor)
     assert np.array_equal(bits16(got), exp.view(np.uint16))
+
+
+@pytest.mark.parametrize("bits", [16, 8, 4])
+@pytest.mark.parametrize("V", [8, 4, 2])
+@pytest.mark.parametrize("layout", ["aligned", "scattered"])
+def test_softmax_edges(bits, V, layout):
+    """P against the restatement with the softmax's own exponentials: rows
+    short, longer than the registers hold (1030 slots), and with sums outside
+    the corrected reciprocal's range (rows v >= 1 far below their maximum's
+    start at 0; an infinite or NaN logit)."""
+    batch, scale = 2, {16: 32767.0, 8: 127.0, 4: 7.0}[bits]
+    order, pairs, cols = ragged_mask(32, seed=V + bits)
+    if layout == "scattered":
+        pairs, cols = scattered(pairs, cols, seed=V)
+    rng = np.random.default_rng(bits * V)
+    logits = (rng.standard_normal((batch, cols.size, V)) * 16).astype(np.float16)
+    low = pairs[2 * 9]                       # the row of 65 slots: exponentials near the smallest float
+    logits[1, low:low + 65] = (-80 * 8 + rng.standard_normal((65, V))).astype(np.float16)
+    real = np.zeros(cols.size, bool)
+    for i in range(pairs.size // 2):
+        real[pairs[2 * i]:pairs[2 * i + 1]] = True
+    logits[:, ~real] = np.float16("nan")     # never read
+    logits = logits.reshape(batch, -1)
+    print(f"softmax bits={bits} V={V} {layout}", flush=True)
+    attn = sptrans.q_bcsr_softmax(dev(order), dev(pairs), dev(logits), 0.125, scale, V, batch, bits)
+    torch.cuda.synchronize()
+    exp = oatt.ref_softmax_f16(logits, pairs, order, V, 0.125, scale, bits)
+    raw = attn.cpu().numpy().view(np.uint8)
+    for b in range(batch):
+        got = oatt.unpack_p_reference(raw[b], cols.size, V, bits)
+        # one step from rounding at a step's edge; 16-bit steps are as fine as
+        # the exponential's own error (a few ulp of 2^-23 times 2^15)
+        assert np.abs(got - exp[b]).max() <= 1
+        assert (got != exp[b]).sum() <= max(4, got.size // 100)
+        assert (got[~real] == 0).all()
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("rows", [(5, 64, 8), (3, 40, 24), (1, 7, 8), (2, 9, 40)])
+def test_quantize_matches_the_restatement(bits, rows):
+    """One tensor, contiguous or not, odd row counts, edges of a thread's and a block's share."""
+    b, n, d = rows
+    x = torch.randn((b, n * 61, d), device="cuda").half()
+    for t in (x, x.transpose(0, 1), x[:, 1:]):
+        if (d * bits) % 32:
+            continue
+        got = sptrans.bquantization(t, bits, 30.0)
+        exp = oatt.quantize_ref(t.contiguous().cpu().numpy(), 30.0, bits, 0)
+        lanes = formats.unpack_lanes(got.cpu().numpy().view(np.uint8), bits, exp.size, signed=True)
+        assert np.array_equal(lanes.reshape(exp.shape), exp)
