@@ -211,7 +211,7 @@ __global__ __launch_bounds__(64 * WPB) void softmax_requant_kernel(int m_vec, co
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int v = 4 * g + i;
-                s[t][i] = (home && i < HOME && slot < end) ? (float)s_vals[(size_t)slot * V + v] * alpha : -INFINITY;
+                s[t][i] = (home && i < HOME && slot < end) ? scaled_logit(s_vals[(size_t)slot * V + v], alpha) : -INFINITY;
             }
         }
     };
@@ -219,17 +219,31 @@ __global__ __launch_bounds__(64 * WPB) void softmax_requant_kernel(int m_vec, co
     float m[HOME], l[HOME];
 #pragma unroll
     for (int i = 0; i < HOME; ++i) { m[i] = -INFINITY; l[i] = 0.f; }
+    float mq[HOME];
+    const bool online = p_mode != kPModeRowScaled && nch > kRowChunks<V>;
     for (int ch = 0; ch < nch; ++ch) {
         float s[4][4];
         load_chunk(ch, s);
-        softmax_chunk_update<HOME>(s, m, l);
+        if (online) softmax_lane_update<HOME>(s, m, l);
+        else softmax_lane_max<HOME>(s, m);
     }
+#pragma unroll
+    for (int i = 0; i < HOME; ++i) mq[i] = finite_row_max(row16_max(m[i]));
+    if (online) {
+#pragma unroll
+        for (int i = 0; i < HOME; ++i) l[i] *= __expf(m[i] - mq[i]);
+    } else {
+        for (int ch = 0; ch < nch; ++ch) {
+            float s[4][4];
+            load_chunk(ch, s);
+            softmax_lane_exp<HOME>(s, mq, l);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < HOME; ++i) l[i] = row16_sum(l[i]);
     float inv_l[HOME];
 #pragma unroll
     for (int i = 0; i < HOME; ++i) inv_l[i] = l[i] > 0.f ? 1.0f / l[i] : 0.f;
-    float mq[HOME];
-#pragma unroll
-    for (int i = 0; i < HOME; ++i) mq[i] = finite_row_max(m[i]);
     if (row_inv_l && home && c == 0) {
 #pragma unroll
         for (int i = 0; i < HOME; ++i) row_inv_l[(size_t)i_row * V + 4 * g + i] = inv_l[i];
@@ -509,54 +523,61 @@ __device__ __forceinline__ int const_load(const int *p) {
 // ---------------------------------------------------------------------------
 // Fused batched attention: persistent waves walk a work list of (matrix,
 // vector row) items.  Pass 1 gathers K rows, computes the int32 logits with
-// MFMA and keeps the online softmax statistics; pass 2 recomputes the exact
-// logits, quantizes P, moves it to the A layout through LDS, gathers V rows
-// (4x4 byte transposes) and accumulates O = P V with MFMA.
+// MFMA and keeps the row maxima; pass 2 quantizes P from one exponential per
+// logit, moves it to the A layout through LDS, gathers V rows (4x4 byte
+// transposes) and accumulates O = P V with MFMA.
 // VB = 4: V rows are packed 4-bit ([L][32] bytes, lane 0 low); each lane
 // gathers the 16 bits of its four columns and widens them to the bytes
 // V + 8 (0..15), so the MFMA forms P (V + 8) and 8 * (row sum of P) comes off
 // the accumulators at the end (exact mod 2^32).
+//
+// Bound by the address and data path of L1 (TA / TD busy three quarters of the
+// kernel) with VALU issue close behind, not by L2: sending every gather to one
+// 4 KB window takes the same time, dropping the arithmetic or the gathers does
+// not.  So each logit is scaled, exponentiated and summed once: pass 1 needs
+// the max alone, its logits go to pass 2 through LDS (the first SST chunks)
+// and registers (two more); lanes keep their own sums, reduced once per row;
+// the real rows sit in all four lane groups of the MFMA tile; four P bytes are
+// written as one dword; K rows are gathered row-contiguous.  Measured, us per
+// launch, before (online softmax per chunk in pass 1, K and P recomputed) and
+// now: 32 matrices of L = 4096, 90 % sparse, V = 8, reference P 96 -> 80;
+// 64 of L ~ U[512, 4096], row-scaled P 84 -> 70; 4 of L = 8192, 80 % sparse
+// 163 -> 145; 16 of L = 4096, 80 % sparse, V = 2 243 -> 204.
 // ---------------------------------------------------------------------------
 // DBG instantiations also write the optional int32 S, int8 P and int32 P V
 // outputs; the production ones carry no stores inside the chunk loops (a
 // conditional store there would make every load wait drain the queue).
-// Pass 2 takes the scaled logits of a row's first chunks from an LDS copy
-// made in pass 1 instead of gathering K and recomputing them: 12 KB per wave
-// (8 floats per lane and chunk at V = 8, so six chunks; 4 and twelve at
-// V = 2 and 4), 52 KB per workgroup with the P tiles, so three workgroups
-// (three waves per SIMD, at most 168 registers) fit a CU's 160 KB.  Measured
-// on 128 matrices of L ~ U[512, 4096]: 0.199 ms per step, against 0.233 ms
-// with no copy at four waves per SIMD, 0.209 ms with a copy of three chunks
-// of K instead, 0.210 ms with 8 KB of logits at four waves.
-constexpr int kLogitStashBytes = 12288;   // per wave
-
+// LDS: 12 KB of logits and a 1 KB P tile per wave, 52 KB per workgroup, so
+// three workgroups (three waves per SIMD, at most 168 registers) fit a CU's
+// 160 KB.
 template <int V, int QKB, int VB, int PM, int WPB, bool DBG>
-__global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(3))) void attention_kernel(const AttnMatrix *mats, const int2 *items, int n_items,
-                                                             float p_scale, int p_mode) {
-    constexpr int HOME = V < 4 ? V : 4;
+__global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(3))) void attention_kernel(
+    const AttnMatrix *mats, const int2 *items, int n_items, float p_scale) {
     constexpr int QROW = kHeadDim * QKB / 8;          // bytes per Q/K row
     constexpr int KCB = QROW / 4;                     // bytes of a K row per lane
     __shared__ __attribute__((aligned(16))) unsigned char tiles[WPB][16 * 64];
     // logits s[t][j] of a row's first SST chunks, kept from pass 1 for pass 2
     // (per wave; SQ 16-byte slots per lane, lane-major, so the accesses are
     // conflict-free)
-    constexpr int HC_ = V == 8 ? 2 : 1;
-    constexpr int SQ = HC_;                       // 4 * HC floats per lane
-    constexpr int SST = kLogitStashBytes / (64 * 16 * SQ);
+    constexpr int SQ = V == 8 ? 2 : 1;            // 4 * HC floats per lane
+    constexpr int SST = kStashChunks<V>;
     __shared__ v4f sstash[WPB][SST][SQ][64];
     // the wave id in an SGPR keeps work-item indices, descriptors and buffer
     // resources wave-uniform (no per-lane waterfall around each buffer load)
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    const bool home = g < (V + 3) / 4;
-    // Softmax rows per lane: the MFMA C tile holds the V real rows in lane
-    // groups g < (V + 3) / 4 (rows 4g + i); permlane swaps deal them to all
-    // four groups first, so that the per-logit work runs on real rows only.
-    // V = 8: group g holds rows row0 + {0, 1}, row0 = 4 (g & 1) + 2 (g >> 1);
-    // V = 4: group g holds row g; V = 2: groups 0 and 1 hold rows 0 and 1.
+    // The V rows sit in the MFMA's row tile at rows 4q + j, j < HC: lane group
+    // g of the C tile then holds vector rows HC * g + j in its first HC
+    // accumulators, so that the per-logit work and the epilogue run on real
+    // rows in every lane without moving any (rows 0..V-1 would leave them in
+    // half the lanes at V = 8 and a quarter at V = 4).  The other tile rows
+    // read Q and P out of range or unwritten and feed nothing.
     constexpr int HC = V == 8 ? 2 : 1;
-    const bool chome = V == 2 ? g < 2 : true;
-    const int row0 = V == 8 ? 4 * (g & 1) + 2 * (g >> 1) : g;
+    constexpr int NCH = kRowChunks<V>;
+    const bool chome = HC * g < V;
+    const int row0 = HC * g;                                  // lane's vector rows row0 + j
+    const int a_row = HC * (c >> 2) + (c & 3);                // vector row of tile row c
+    const bool a_live = (c & 3) < HC && a_row < V;
     const int nwaves = gridDim.x * WPB;
 
     for (int it = blockIdx.x * WPB + wave; it < n_items; it += nwaves) {
@@ -588,7 +609,6 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(3))) v
                   end = uniform(const_load(M.row_offsets + 2 * i_row + 1));
         const int aend = start + ((end - start + 15) & ~15);
         const int nch = (end - start + 63) >> 6;
-        const int nch_w = (aend - start + 63) >> 6;
         const u32 kv_bytes = (u32)M.L * QROW;
         const __amdgpu_buffer_rsrc_t rk = make_rsrc(M.k, kv_bytes);
         const __amdgpu_buffer_rsrc_t rv = make_rsrc(M.v, (u32)M.L * (kHeadDim * VB / 8));
@@ -599,15 +619,15 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(3))) v
         // fp16 Q (q16 non-null): lane (c, g) loads columns 16g .. 16g + 15
         // of row i_row * V + c here and quantizes them once the pipeline's
         // first index and K loads are out (quantize_q16)
-        v4i qh0, qh1;
+        v4i qh0 = v4i{0, 0, 0, 0}, qh1 = v4i{0, 0, 0, 0};
         if (M.q16) {
             const __amdgpu_buffer_rsrc_t rq16 =
                 make_rsrc(M.q16, (u32)(((u32)(M.L - 1) * (u32)M.q16_stride + kHeadDim) * 2u));
-            const u32 off = c < V ? ((u32)(i_row * V + c) * (u32)M.q16_stride + (u32)(16 * g)) * 2u : 0x80000000u;
+            const u32 off = a_live ? ((u32)(i_row * V + a_row) * (u32)M.q16_stride + (u32)(16 * g)) * 2u : 0x80000000u;
             qh0 = buf_load_b128(rq16, off);
             qh1 = buf_load_b128(rq16, off + 16u);
         } else {
-            const u32 off = c < V ? (u32)(i_row * V + c) * QROW + (u32)(16 * g * QKB / 8) : 0x80000000u;
+            const u32 off = a_live ? (u32)(i_row * V + a_row) * QROW + (u32)(16 * g * QKB / 8) : 0x80000000u;
             qop = load_k16<QKB>(rq, off);
             if constexpr (QKB == 4) qop = expand_nibbles(qop, true, 0u);
         }
@@ -633,34 +653,141 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(3))) v
             else qop = v4i{pack(0, 2, 4, 6), pack(1, 3, 5, 7), pack(8, 10, 12, 14), pack(9, 11, 13, 15)};
         };
 
-        // ---- software pipeline over 64-slot chunks.  Per half step for chunk
-        // ch: issue the index load of chunk ch+2, the row gathers of chunk ch+1
-        // (its index arrived one half step ago), then consume chunk ch.  Loads
-        // retire in order, so each consumer waits only for older loads and the
-        // gathers of the next chunk stay in flight.  Chunks past the row end
-        // are fully masked: they leave (m, l) bitwise unchanged and add P = 0,
-        // so the loops run in pairs without branches.
         const __amdgpu_buffer_rsrc_t rc = make_rsrc(M.col_indices, 0x7FFFFFFFu);
+        constexpr u32 kRowOob = 0x80000000u;
+        // ---- the row.  The first SST chunks' logits are kept in LDS, and two
+        // more in registers where that is the whole row (nch <= NCH): then K
+        // is gathered once, the max and sum are reduced across lanes once and
+        // every exponential is taken once.  Later chunks of longer rows are
+        // gathered and multiplied again for their P.  Slot order: lane
+        // 16g + p of an index load holds slot 16 (p % 4) + 4g + p / 4 of its
+        // chunk, so that P packs four slots 16t + c per dword (t the byte) on
+        // its way to the A layout while V offsets still come from the lane's
+        // own row of 16.
+        // Per half step for chunk ch: the index load of chunk ch + 2 and the
+        // row gathers of chunk ch + 1 go out before chunk ch is consumed.
+        // Loads retire in order, so each consumer waits only for older loads.
+        const bool kept = nch <= NCH;
+        const int pslot = 16 * (lane & 3) + 4 * g + ((lane >> 2) & 3);
+        const int perm_addr = 4 * (4 * c + g);
         // per lane: byte offset of its slot's V row (index * 64), or the
         // out-of-range marker for slots past the row end (L * 64 < 2^31)
-        constexpr u32 kRowOob = 0x80000000u;
         auto load_idx = [&](int ch) {
-            const int slot = start + 64 * ch + lane;
+            const int slot = start + 64 * ch + pslot;
             const u32 v = buf_load_b32(rc, slot < end ? (u32)slot * 4u : kRowOob);
             return slot < end ? v * (u32)kHeadDim : kRowOob;
         };
-        // K rows of slots 16t + c, bytes [KCB * g, +KCB): the MFMA B operand
-        // directly (gathering four lanes per row and moving the rows to this
-        // layout through LDS makes fewer L1 accesses but measured slower)
+        // K rows of a tile, row-contiguous: lane 4i + j holds piece j of slot
+        // 16t + i's row (16 L1 accesses for 16 rows; gathered in the operand
+        // layout, 16 rows per 16 lanes, a load makes 64).  The row offset is
+        // lane t of the lane's quad.  logits() moves the data to the operand
+        // layout with one ds_bpermute per dword.
         auto load_krows = [&](u32 my_off, v4i (&kop)[4]) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                u32 row = (u32)__shfl((int)my_off, 16 * t + c, 64);
+                u32 row = (u32)quad_bcast((int)my_off, t);
                 if constexpr (QKB == 4) row = (row >> 1) | (row & kRowOob);   // 32-byte rows, marker kept
-                kop[t] = load_k16<QKB>(rk, row + (u32)(KCB * g));
+                kop[t] = load_k16<QKB>(rk, row + (u32)(KCB * (lane & 3)));
             }
         };
-        // V rows of slots 16g + p (p = 0..15), columns 4c..4c+3: dword c of an
+        auto put = [&](int ch, const float (&s)[4][HC]) {
+#pragma unroll
+            for (int q = 0; q < SQ; ++q) {
+                v4f x;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = s[(4 * q + e) / HC][(4 * q + e) % HC];
+                sstash[wave][ch][q][lane] = x;
+            }
+        };
+        auto get = [&](int ch, float (&s)[4][HC]) {
+#pragma unroll
+            for (int q = 0; q < SQ; ++q) {
+                const v4f x = sstash[wave][ch][q][lane];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[(4 * q + e) / HC][(4 * q + e) % HC] = x[e];
+            }
+        };
+        // scaled logits of one chunk
+        auto logits = [&](int ch, const v4i (&kop)[4], float (&s)[4][HC]) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                v4i kk = row_to_operand<QKB == 4 ? 2 : 4>(kop[t], perm_addr);
+                if constexpr (QKB == 4) kk = expand_nibbles(kk, true, 0u);
+                const v4i acc = mfma_i8(qop, kk, v4i{0, 0, 0, 0});
+                if constexpr (DBG) {
+                    const int slot = start + 64 * ch + 16 * t + c;
+                    if (M.s_out && chome && slot < end) {
+#pragma unroll
+                        for (int j = 0; j < HC; ++j) M.s_out[(size_t)slot * V + row0 + j] = acc[j];
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < HC; ++j) s[t][j] = scaled_logit(acc[j], M.alpha);
+            }
+            if (ch >= nch - 1) {     // only the row's last chunk has masked slots
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int j = 0; j < HC; ++j) s[t][j] = start + 64 * ch + 16 * t + c < end ? s[t][j] : -INFINITY;
+            }
+        };
+        float m[HC], l[HC], inv_l[HC], mq[HC];
+#pragma unroll
+        for (int j = 0; j < HC; ++j) { m[j] = -INFINITY; l[j] = 0.f; inv_l[j] = 0.f; }
+        // the running statistics after one chunk's logits
+        auto update = [&](const float (&s)[4][HC]) {
+            if (PM != kPModeRowScaled && !kept) softmax_lane_update<HC>(s, m, l);
+            else softmax_lane_max<HC>(s, m);
+        };
+        float sreg[2][4][HC];
+        const u32 off0 = load_idx(0), off1 = load_idx(1);
+        u32 ia = off0, ib = off1;
+        {
+            v4i ka[4], kb[4];
+            float s[4][HC];
+            load_krows(ia, ka);
+            if (M.q16) quantize_q16();
+            for (int ch = 0; ch < SST; ch += 2) {
+                if (ch >= nch) break;
+                ia = load_idx(ch + 2);
+                load_krows(ib, kb);
+                logits(ch, ka, s);
+                put(ch, s);
+                update(s);
+                __builtin_amdgcn_sched_barrier(0);
+                if (ch + 1 >= nch) break;
+                ib = load_idx(ch + 3);
+                load_krows(ia, ka);
+                logits(ch + 1, kb, s);
+                put(ch + 1, s);
+                update(s);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (nch > SST) {
+                if (kept) {
+                    load_krows(ib, kb);
+                    logits(SST, ka, sreg[0]);
+                    softmax_lane_max<HC>(sreg[0], m);
+                    logits(SST + 1, kb, sreg[1]);
+                    softmax_lane_max<HC>(sreg[1], m);
+                } else {
+                    for (int ch = SST; ch < nch; ch += 2) {
+                        ia = load_idx(ch + 2);
+                        load_krows(ib, kb);
+                        logits(ch, ka, s);
+                        update(s);
+                        __builtin_amdgcn_sched_barrier(0);
+                        ib = load_idx(ch + 3);
+                        load_krows(ia, ka);
+                        logits(ch + 1, kb, s);
+                        update(s);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+        }
+        // V rows of slots in pslot order: lane 16g + p of the index load holds
+        // byte p of the lane group's A operand; columns 4c..4c+3: dword c of an
         // int8 row, or the 16 bits at byte 2c of a packed 4-bit row
         auto load_vrows = [&](u32 my_off, u32 (&raw)[16]) {
 #pragma unroll
@@ -674,115 +801,75 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(3))) v
                 }
             }
         };
-        // C-tile rows 4g + i of one 16-slot tile -> this lane's rows row0 + j
-        auto compact_rows = [&](const v4i &acc, int (&out)[HC]) {
-            if constexpr (V == 8) {
-                // lanes 32..63 take rows 4g' + 2, 4g' + 3 of lanes 0..31 (g' = g - 2)
-                out[0] = (int)__builtin_amdgcn_permlane32_swap((u32)acc[0], (u32)acc[2], false, false)[0];
-                out[1] = (int)__builtin_amdgcn_permlane32_swap((u32)acc[1], (u32)acc[3], false, false)[0];
-            } else if constexpr (V == 4) {
-                // rows 0, 1 to groups 0, 1 and rows 2, 3 to groups 2, 3
-                const u32 a = __builtin_amdgcn_permlane16_swap((u32)acc[0], (u32)acc[1], false, false)[0];
-                const u32 b = __builtin_amdgcn_permlane16_swap((u32)acc[2], (u32)acc[3], false, false)[0];
-                out[0] = (int)__builtin_amdgcn_permlane32_swap(a, b, false, false)[0];
+        // V of the first chunk is in flight while the statistics finish
+        ib = off1;
+        u32 va[16], vb[16];
+        load_vrows(off0, va);
+#pragma unroll
+        for (int j = 0; j < HC; ++j) mq[j] = finite_row_max(row16_max(m[j]));
+        if constexpr (PM != kPModeRowScaled) {
+            // P needs the row sum
+            if (kept) {
+                for (int ch = 0; ch < SST; ++ch) {
+                    if (ch >= nch) break;
+                    float s[4][HC];
+                    get(ch, s);
+                    softmax_lane_exp<HC>(s, mq, l);
+                    put(ch, s);
+                }
+                if (nch > SST) {
+                    softmax_lane_exp<HC>(sreg[0], mq, l);
+                    softmax_lane_exp<HC>(sreg[1], mq, l);
+                }
             } else {
-                out[0] = (int)__builtin_amdgcn_permlane16_swap((u32)acc[0], (u32)acc[1], false, false)[0];
+#pragma unroll
+                for (int j = 0; j < HC; ++j) l[j] *= __expf(m[j] - mq[j]);
             }
-        };
-        // logits of one chunk, scaled, in this lane's rows; masked -> -inf.
-        // si: the raw C tile (rows 4g + i), kept for the debug outputs only
-        auto logits = [&](int ch, const v4i (&kop)[4], float (&s)[4][HC], int (&si)[4][4]) {
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                v4i kk = kop[t];
-                if constexpr (QKB == 4) kk = expand_nibbles(kk, true, 0u);
-                const v4i acc = mfma_i8(qop, kk, v4i{0, 0, 0, 0});
-                const int slot = start + 64 * ch + 16 * t + c;
-                if constexpr (DBG) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) si[t][i] = acc[i];
-                }
-                int v[HC];
-                compact_rows(acc, v);
-#pragma unroll
-                for (int j = 0; j < HC; ++j) s[t][j] = (chome && slot < end) ? (float)v[j] * M.alpha : -INFINITY;
-            }
-        };
-
-        float m[HC], l[HC];
-#pragma unroll
-        for (int j = 0; j < HC; ++j) { m[j] = -INFINITY; l[j] = 0.f; }
-        auto pass1_chunk = [&](int ch, const v4i (&kop)[4]) {
-            float s[4][HC];
-            int si[4][4];
-            logits(ch, kop, s, si);
-            if (ch < SST) {
-#pragma unroll
-                for (int q = 0; q < SQ; ++q) {
-                    v4f x;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x[e] = s[(4 * q + e) / HC][(4 * q + e) % HC];
-                    sstash[wave][ch][q][lane] = x;
-                }
-            }
-            softmax_chunk_update<HC>(s, m, l);
-            if (DBG && M.s_out && home) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const int slot = start + 64 * ch + 16 * t + c;
-#pragma unroll
-                    for (int i = 0; i < HOME; ++i)
-                        if (slot < end) M.s_out[(size_t)slot * V + 4 * g + i] = si[t][i];
-                }
-            }
-        };
-        {
-            v4i ka[4], kb[4];
-            u32 ia = load_idx(0);
-            u32 ib = load_idx(1);
-            load_krows(ia, ka);
-            if (M.q16) quantize_q16();
-            for (int ch = 0; ch < nch; ch += 2) {
-                ia = load_idx(ch + 2);
-                load_krows(ib, kb);
-                pass1_chunk(ch, ka);
-                __builtin_amdgcn_sched_barrier(0);
-                ib = load_idx(ch + 3);
-                load_krows(ia, ka);
-                pass1_chunk(ch + 1, kb);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int j = 0; j < HC; ++j) {
+                l[j] = row16_sum(l[j]);
+                inv_l[j] = l[j] > 0.f ? 1.0f / l[j] : 0.f;
             }
         }
-        float inv_l[HC];
-#pragma unroll
-        for (int j = 0; j < HC; ++j) inv_l[j] = l[j] > 0.f ? 1.0f / l[j] : 0.f;
-        float mq[HC];
-#pragma unroll
-        for (int j = 0; j < HC; ++j) mq[j] = finite_row_max(m[j]);
-
         v4i oacc[4];
 #pragma unroll
         for (int b = 0; b < 4; ++b) oacc[b] = v4i{0, 0, 0, 0};
-        int psum = 0;   // VB = 4: sum of P row c over this lane's slots 16g..16g+15 of every chunk
-        auto pass2_chunk = [&](int ch, const v4i (&kop)[4], const u32 (&raw_in)[16]) {
-            float s[4][HC];
-            int si[4][4];
-            if (ch < SST) {
-#pragma unroll
-                for (int q = 0; q < SQ; ++q) {
-                    const v4f x = sstash[wave][ch][q][lane];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) s[(4 * q + e) / HC][(4 * q + e) % HC] = x[e];
-                }
+        int psum = 0;   // VB = 4: sum of P row c over this lane's slots of every chunk
+        // exponentials and 1 / sum are at most 1: only a scale above 127 (or the
+        // 4-bit mode) can exceed P's range
+        const bool clamp = PM == kPModeReference4 || p_scale > 127.f;
+        // O += P V of one chunk; s: its logits, or (reference modes, kept
+        // rows) its exponentials
+        auto output = [&](int ch, float (&s)[4][HC], const u32 (&raw_in)[16]) {
+            if constexpr (PM == kPModeRowScaled) {
+                softmax_lane_exp<HC>(s, mq, l);
             } else {
-                logits(ch, kop, s, si);
+                if (!kept) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int j = 0; j < HC; ++j) s[t][j] = __expf(s[t][j] - mq[j]);
+                }
             }
-            int pq[4][HC];
+            u32 pq[HC];
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int j = 0; j < HC; ++j) {
+                u32 b[4];
 #pragma unroll
-                for (int j = 0; j < HC; ++j) pq[t][j] = quantize_prob<PM>(s[t][j], mq[j], inv_l[j], p_scale, p_mode);
-            const v4i pop = p_to_a_layout<HC>(tiles[wave], pq, lane, chome, row0);
+                for (int t = 0; t < 4; ++t) b[t] = quantize_exp_byte<PM>(s[t][j], inv_l[j], p_scale, clamp);
+                pq[j] = perm(perm(b[3], b[2], 0x0C0C0400u), perm(b[1], b[0], 0x0C0C0400u), 0x05040100u);
+            }
+            const v4i pop = p_dwords_to_a_layout<HC>(tiles[wave], pq, lane, chome);
+            if (DBG && M.p_out && a_live) {
+                // byte b of the lane: row a_row, slot 16 (b % 4) + 4g + b / 4
+#pragma unroll
+                for (int b = 0; b < 16; ++b) {
+                    const int slot = start + 64 * ch + 16 * (b & 3) + 4 * g + (b >> 2);
+                    if (slot < aend)
+                        M.p_out[(size_t)(slot >> 4) * 16 * V + 16 * a_row + (slot & 15)] =
+                            (unsigned char)((u32)pop[b >> 2] >> (8 * (b & 3)));
+                }
+            }
             u32 raw[16];
 #pragma unroll
             for (int p = 0; p < 16; ++p) {
@@ -795,11 +882,6 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(3))) v
                 }
             }
             if constexpr (VB == 4) psum += sum_bytes(pop);
-            if (DBG && M.p_out) {
-                const int slot0 = start + 64 * ch + 16 * g;
-                if (c < V && slot0 < aend)
-                    *reinterpret_cast<v4i *>(M.p_out + (size_t)(slot0 >> 4) * 16 * V + 16 * c) = pop;
-            }
             // after the 4x4 byte transposes, tr[q][b] holds column 4c + b of rows 4q..4q+3
             u32 tr[4][4];
 #pragma unroll
@@ -811,64 +893,77 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(3))) v
             }
         };
         {
-            // the first SST chunks' logits come from pass 1's LDS copy (the
-            // same values pass 2 would recompute), the rest from K gathered
-            // again
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            auto get_krows = [&](int ch, u32 my_off, v4i (&kop)[4]) {
-                if (ch >= SST) load_krows(my_off, kop);
-            };
-            v4i ka[4], kb[4];
-            u32 va[16], vb[16];
-            u32 ia = load_idx(0);
-            u32 ib = load_idx(1);
-            get_krows(0, ia, ka);
-            load_vrows(ia, va);
-            for (int ch = 0; ch < nch_w; ch += 2) {
+            float s[4][HC];
+            for (int ch = 0; ch < SST; ch += 2) {
+                if (ch >= nch) break;
                 ia = load_idx(ch + 2);
-                get_krows(ch + 1, ib, kb);
                 load_vrows(ib, vb);
-                pass2_chunk(ch, ka, va);
+                get(ch, s);
+                output(ch, s, va);
                 __builtin_amdgcn_sched_barrier(0);
+                if (ch + 1 >= nch) break;
                 ib = load_idx(ch + 3);
-                get_krows(ch + 2, ia, ka);
                 load_vrows(ia, va);
-                pass2_chunk(ch + 1, kb, vb);
+                get(ch + 1, s);
+                output(ch + 1, s, vb);
                 __builtin_amdgcn_sched_barrier(0);
             }
+            if (nch > SST) {
+                if (kept) {
+                    load_vrows(ib, vb);
+                    output(SST, sreg[0], va);
+                    output(SST + 1, sreg[1], vb);
+                } else {
+                    // ia, ib: chunks SST and SST + 1; va: chunk SST
+                    v4i ka[4], kb[4];
+                    load_krows(ia, ka);
+                    for (int ch = SST; ch < nch; ch += 2) {
+                        ia = load_idx(ch + 2);
+                        load_krows(ib, kb);
+                        load_vrows(ib, vb);
+                        logits(ch, ka, s);
+                        output(ch, s, va);
+                        __builtin_amdgcn_sched_barrier(0);
+                        ib = load_idx(ch + 3);
+                        load_krows(ia, ka);
+                        load_vrows(ia, va);
+                        logits(ch + 1, kb, s);
+                        output(ch + 1, s, vb);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
         }
-        // 1 / row sum of output rows 4g + i, from the lanes that hold those rows
-        float row_inv_l[HOME];
+        if constexpr (PM == kPModeRowScaled) {
 #pragma unroll
-        for (int i = 0; i < HOME; ++i) {
-            const int src_group = V == 8 ? (g | (i & 2)) : ((4 * g + i) & 3);
-            row_inv_l[i] = __shfl(inv_l[V == 8 ? (i & 1) : 0], 16 * src_group + c, 64);
+            for (int j = 0; j < HC; ++j) {
+                l[j] = row16_sum(l[j]);
+                inv_l[j] = l[j] > 0.f ? 1.0f / l[j] : 0.f;
+            }
         }
         if constexpr (VB == 4) {
-            // row c's sum of P over all slots (the four lane groups hold
-            // slots 16g..16g+15 of every chunk), then 8 * sum(P) of output
-            // row 4g + i off its accumulators
+            // tile row c's sum of P over all slots (the four lane groups hold
+            // a quarter of every chunk each), then 8 * sum(P) of tile row
+            // 4g + j off its accumulators
             int s = psum;
             s += lane_read(s, lane ^ 16);
             s += lane_read(s, lane ^ 32);
 #pragma unroll
-            for (int i = 0; i < HOME; ++i) {
+            for (int i = 0; i < HC; ++i) {
                 const u32 corr = 8u * (u32)lane_read(s, 4 * g + i);
 #pragma unroll
                 for (int b = 0; b < 4; ++b) oacc[b][i] = (int)((u32)oacc[b][i] - corr);
             }
         }
-        // rows 4g+i, columns 4c + b
-        if (home) {
+        // rows row0 + i, columns 4c + b
+        if (chome) {
 #pragma unroll
-            for (int i = 0; i < HOME; ++i) {
-                const size_t orow = (size_t)(i_row * V + 4 * g + i) * kHeadDim + 4 * c;
+            for (int i = 0; i < HC; ++i) {
+                const size_t orow = (size_t)(i_row * V + row0 + i) * kHeadDim + 4 * c;
                 if (DBG && M.o_int)
                     *reinterpret_cast<v4i *>(M.o_int + orow) = v4i{oacc[0][i], oacc[1][i], oacc[2][i], oacc[3][i]};
                 // same float operations as dequant_kernel with/without a row scale
-                const float rs = PM == kPModeRowScaled ? row_inv_l[i] : 1.f;
+                const float rs = PM == kPModeRowScaled ? inv_l[i] : 1.f;
                 float4 of;
                 of.x = ((float)oacc[0][i] * M.o_scale) * rs;
                 of.y = ((float)oacc[1][i] * M.o_scale) * rs;
@@ -879,7 +974,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(3))) v
                     // [L][row stride] layout, e.g. the [L][batch][heads * 64]
                     // input of the output projection
                     const __half2 h01 = __floats2half2_rn(of.x, of.y), h23 = __floats2half2_rn(of.z, of.w);
-                    const size_t hrow = (size_t)(i_row * V + 4 * g + i) * (size_t)M.o16_stride + 4 * c;
+                    const size_t hrow = (size_t)(i_row * V + row0 + i) * (size_t)M.o16_stride + 4 * c;
                     *reinterpret_cast<v2i *>(M.o16 + hrow) =
                         v2i{*reinterpret_cast<const int *>(&h01), *reinterpret_cast<const int *>(&h23)};
                 } else {
@@ -1046,10 +1141,10 @@ mc_status mc_attn_forward(const mc_attn_matrix *matrices, const int *items, int 
     do {                                                                                                             \
         if (debug)                                                                                                   \
             hipLaunchKernelGGL((mc::attention_kernel<V_, B_, VB_, PM_, WPB, true>), grid, block, 0, stream, mats,    \
-                               its, n_items, p_scale, p_mode);                                                       \
+                               its, n_items, p_scale);                                                               \
         else                                                                                                         \
             hipLaunchKernelGGL((mc::attention_kernel<V_, B_, VB_, PM_, WPB, false>), grid, block, 0, stream, mats,   \
-                               its, n_items, p_scale, p_mode);                                                       \
+                               its, n_items, p_scale);                                                               \
     } while (0)
 #define MC_ATTN_LAUNCH_P(V_, B_, VB_)                                                                                \
     switch (p_mode) {                                                                                                \

@@ -15,12 +15,15 @@
 // Rows are the V matrix rows of one vector row; max/sum run over the row's
 // nonzero slots.
 //
-// Canonical softmax statistics: a row's slots are visited in chunks of 64
-// (four 16-slot MFMA tiles, slot order).  Per chunk: exact max M_c; running
-// max m' = max(m, M_c); lane c first adds its four slots c, 16 + c, 32 + c,
-// 48 + c as (e0 + e1) + (e2 + e3), then the 16 lane sums are added as a
-// pairwise tree over lane order; running sum l = l * exp(m - m') + chunk sum.  Both kernels evaluate these statistics
-// on the same register layout (MFMA C layout: lane (c, g) holds rows 4g+i of
+// Canonical softmax statistics: the exact max m over the row; lane c of 16
+// adds exp(s - m) of its slots chunk by chunk of 64 (four 16-slot MFMA tiles,
+// slot order), (e0 + e1) + (e2 + e3) of the slots c, 16 + c, 32 + c, 48 + c of
+// a chunk at a time, then the 16 lane sums are added as a pairwise tree over
+// lane order.  Rows of more than kRowChunks chunks whose P needs the sum (the
+// reference modes) are not visited a third time: there each lane keeps the
+// sum against its own running max, rescaled when that grows, and brings it to
+// the row max before the tree.  Both kernels evaluate these statistics on the
+// same register layout (MFMA C layout: lane (c, g) holds rows 4g+i of
 // slot 16t + c) with the same instructions.  The fused kernel first moves
 // the V real rows out of the MFMA tile's padding lanes (rows are dealt to
 // the four 16-lane groups instead of four rows per group), so it keeps fewer
@@ -34,6 +37,13 @@
 namespace mc {
 
 constexpr int kHeadDim = 64;
+
+// Chunks of 64 slots whose logits the fused kernel holds: its LDS copy
+// (kLogitStashBytes per wave: six chunks at V = 8, twelve at V = 2 and 4) and
+// two more in registers.
+constexpr int kLogitStashBytes = 12288;   // per wave
+template <int V> constexpr int kStashChunks = kLogitStashBytes / (64 * 16 * (V == 8 ? 2 : 1));
+template <int V> constexpr int kRowChunks = kStashChunks<V> + 2;
 
 // Butterfly reductions within each 16-lane row of the wave, on DPP lane
 // moves (no LDS round trip): swap neighbours, swap pairs (quad_perm), then
@@ -64,25 +74,48 @@ __device__ __forceinline__ float row16_sum(float x) {
     return x;
 }
 
-// Online statistics of one chunk for the HOME rows held by this lane.
+// A logit scaled and rounded by itself: a following subtraction of the row
+// max is never contracted with it, whichever way the value reaches it.
+__device__ __forceinline__ float scaled_logit(int v, float alpha) {
+#pragma clang fp contract(off)
+    return (float)v * alpha;
+}
+
+// max of two values that are no NaN, in one instruction: fmaxf first quiets
+// each input that comes through a branch or memory.
+__device__ __forceinline__ float max2(float a, float b) { return __builtin_amdgcn_fmed3f(a, b, INFINITY); }
+
 // s[t][i]: scaled logit of slot 16t + c for the lane's row i (-inf when masked).
 template <int HOME, int W>
-__device__ __forceinline__ void softmax_chunk_update(const float (&s)[4][W], float (&m)[HOME], float (&l)[HOME]) {
+__device__ __forceinline__ void softmax_lane_max(const float (&s)[4][W], float (&m)[HOME]) {
     static_assert(HOME <= W, "rows held per lane");
 #pragma unroll
+    for (int i = 0; i < HOME; ++i) m[i] = max2(m[i], max2(max2(s[0][i], s[1][i]), max2(s[2][i], s[3][i])));
+}
+// exp(s - m) of one chunk in place (m finite; a masked slot gives exactly 0),
+// and its part of the lane sums.
+template <int HOME, int W>
+__device__ __forceinline__ void softmax_lane_exp(float (&s)[4][W], const float (&m)[HOME], float (&l)[HOME]) {
+#pragma unroll
     for (int i = 0; i < HOME; ++i) {
-        float cm = fmaxf(fmaxf(s[0][i], s[1][i]), fmaxf(s[2][i], s[3][i]));
-        cm = row16_max(cm);
-        const float mn = fmaxf(m[i], cm);        // -inf only while every slot so far is masked
-        // masked slots give exp(-inf) = 0 exactly; the offset is 0 rather
-        // than -inf while the row has no slot yet (-inf - -inf would be NaN)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s[t][i] = __expf(s[t][i] - m[i]);
+        l[i] += (s[0][i] + s[1][i]) + (s[2][i] + s[3][i]);
+    }
+}
+// The lane's running max and its sum against that max after one chunk.  The
+// offset is 0 while the lane has no slot yet (-inf - -inf would be NaN); its
+// sum is 0 then.
+template <int HOME, int W>
+__device__ __forceinline__ void softmax_lane_update(const float (&s)[4][W], float (&m)[HOME], float (&l)[HOME]) {
+#pragma unroll
+    for (int i = 0; i < HOME; ++i) {
+        const float mn = max2(m[i], max2(max2(s[0][i], s[1][i]), max2(s[2][i], s[3][i])));
         const float mz = mn == -INFINITY ? 0.f : mn;
         float e[4];
 #pragma unroll
         for (int t = 0; t < 4; ++t) e[t] = __expf(s[t][i] - mz);
-        const float csum = row16_sum((e[0] + e[1]) + (e[2] + e[3]));
-        const float scale_old = (m[i] == -INFINITY) ? 0.f : __expf(m[i] - mn);
-        l[i] = l[i] * scale_old + csum;
+        l[i] = l[i] * __expf(m[i] - mz) + ((e[0] + e[1]) + (e[2] + e[3]));
         m[i] = mn;
     }
 }
@@ -96,17 +129,28 @@ __device__ __forceinline__ float finite_row_max(float m) { return m == -INFINITY
 
 // Quantized probability of one logit given the final row statistics
 // (m from finite_row_max); a masked slot (s = -inf) gives exp(-inf) = 0.
-// PM fixed at compile time (the fused kernel's chunk loops), or -1 for a
-// run-time p_mode; both evaluate the same expressions.
-template <int PM = -1>
 __device__ __forceinline__ int quantize_prob(float s, float m, float inv_l, float p_scale, int p_mode) {
-    const int mode = PM >= 0 ? PM : p_mode;
     const float e = __expf(s - m);
-    if (mode != kPModeRowScaled)   // truncation (p >= 0)
-        return (int)fminf(e * inv_l * p_scale, mode == kPModeReference4 ? 7.f : 127.f);
+    if (p_mode != kPModeRowScaled)   // truncation (p >= 0)
+        return (int)fminf(e * inv_l * p_scale, p_mode == kPModeReference4 ? 7.f : 127.f);
     return (int)rintf(fminf(e * p_scale, 127.f));
 }
-
+// The same value from the exponential, the mode fixed at compile time (the
+// fused kernel's chunk loops), as the low byte of the result (the other bytes
+// undefined).
+// Without `clamp` (exponential and 1 / sum at most 1, p_scale at most 127) the
+// value cannot exceed 127; adding 1.5 * 2^23 rounds to the nearest integer
+// (ties to even, as rintf) and leaves it in the low bits.
+template <int PM>
+__device__ __forceinline__ u32 quantize_exp_byte(float e, float inv_l, float p_scale, bool clamp) {
+    float t = PM == kPModeRowScaled ? e * p_scale : e * inv_l * p_scale;
+    if (clamp) t = fminf(t, PM == kPModeReference4 ? 7.f : 127.f);
+    if constexpr (PM == kPModeRowScaled) {
+#pragma clang fp contract(off)
+        return __float_as_uint(t + 12582912.f);
+    }
+    return (u32)(int)t;
+}
 
 // Moves P from the lanes' row layout (lane (c, g): rows row0 + i of slot
 // 16t + c; row0 = 4g in the MFMA C layout) to the MFMA A layout (lane (r, g):
@@ -129,6 +173,28 @@ __device__ __forceinline__ v4i p_to_a_layout(unsigned char *tile, const int (&pq
     // above this read).  Workgroup scope would also wait for every gather in
     // flight that lands in LDS.  Rows >= V are never written and only feed
     // output rows that are discarded.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const v4i a = *reinterpret_cast<const v4i *>(tile + c * 64 + 16 * g);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return a;
+}
+
+// The same move with each lane's four slots 16t + c of a row packed in one
+// dword (byte t), the lane's rows at tile rows 4g + i: lane (r, g) gets tile
+// row r, byte b = slot 16 (b % 4) + 4g + b / 4.
+// Two dword writes per lane (V = 8) instead of eight byte writes.
+template <int HOME>
+__device__ __forceinline__ v4i p_dwords_to_a_layout(unsigned char *tile, const u32 (&pq)[HOME], int lane, bool home) {
+    const int c = lane & 15, g = lane >> 4;
+    if (home) {
+#pragma unroll
+        for (int i = 0; i < HOME; ++i) *reinterpret_cast<u32 *>(tile + (4 * g + i) * 64 + 4 * c) = pq[i];
+    }
+    // wavefront-scope fences, as above
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");

@@ -159,6 +159,16 @@ __device__ __forceinline__ int lane_down(int x, int delta) {
     const int lane = __lane_id();
     return __builtin_amdgcn_ds_bpermute(((lane + delta) & 63) << 2, x);
 }
+// Lane t of each quad of lanes, broadcast to the quad (DPP quad_perm); t must
+// fold to a constant.
+__device__ __forceinline__ int quad_bcast(int x, int t) {
+    switch (t & 3) {
+    case 0: return __builtin_amdgcn_update_dpp(0, x, 0x00, 0xF, 0xF, true);
+    case 1: return __builtin_amdgcn_update_dpp(0, x, 0x55, 0xF, 0xF, true);
+    case 2: return __builtin_amdgcn_update_dpp(0, x, 0xAA, 0xF, 0xF, true);
+    default: return __builtin_amdgcn_update_dpp(0, x, 0xFF, 0xF, 0xF, true);
+    }
+}
 // Lane p of each row of 16 lanes, broadcast to that row (DPP row_newbcast,
 // no LDS traffic); p must fold to a constant.
 __device__ __forceinline__ int row_bcast16(int x, int p) {
