@@ -6,7 +6,31 @@
 namespace mc {
 namespace {
 
-int default_config(int rhs_bits, int n, long long m_vec) {
+// MFMA rows of a vector row: its digit planes times its V rows (the planes of
+// the pairs in spmm_kernel.hpp).
+int mfma_rows(int lhs_bits, int rhs_bits, bool sgn, int V) {
+    if (lhs_bits == 4) return V;
+    if (lhs_bits == 8) return (sgn ? 1 : 2) * V;
+    return (lhs_bits / 4 - (sgn ? 1 : 0)) * V;
+}
+
+int default_config(int rhs_bits, int n, long long m_vec, int rows) {
+    // Four dwords of 8- or 16-bit B per lane where the launch fills the GPU
+    // with such tiles (2048 waves of 16 * 4 dwords) and a vector row is one MFMA row tile
+    // (two need 128 accumulators and leave two waves per SIMD).  The gathers
+    // are bound by L1's address path: a 4-byte load of a wave takes it 8
+    // cycles, a 16-byte one 16.  Measured on MI355X, us, one dword and four
+    // waves per row (config 17) against this: L8-R8, V = 8, 8192 x 8192, N =
+    // 4096, 90 % sparse 261 / 160; 4096 x 4096, N = 4096, 70, 90, 98 % 147 /
+    // 112, 59 / 45, 20.3 / 19.4; N = 2048, 90 % 33.5 / 25.6; N = 1024, 70, 90,
+    // 98 % 43 / 32, 16.8 / 14.6, 7.9 / 8.1; N = 512 (1024 waves) 24.0 / 25.2,
+    // 10.1 / 11.7, 6.4 / 6.9.  L16-R8, V = 4, N = 4096, 80 and 95 % 103 / 74,
+    // 32 / 30; L16-R16, V = 4 252 / 154, 77 / 61.  Two row tiles: L16-R8, V =
+    // 8 114 / 135, 42 / 62 (config 25: 99, 55).
+    if (rhs_bits != 4 && rows <= 16 && n % 4 == 0 && n >= 4 * (32 / rhs_bits)) {
+        const int wide = 64 * (32 / rhs_bits);
+        if (m_vec * 2 * ((n + 2 * wide - 1) / (2 * wide)) >= 2048 && n > wide) return 24;
+    }
     // One dword of B per lane and one k-block of gathers in flight per wave:
     // latency is hidden by more resident waves rather than deeper per-wave
     // pipelines.  Up to four waves share a row (one per 16 * 32/bits
@@ -73,17 +97,17 @@ mc_status spmm_entry(int lhs_bits, int rhs_bits, mc_signedness sign, int config,
     if (!row_offsets || !column_indices || !values || !rhs_matrix || !(output_matrix || out16)) return MC_EINVAL_ARG;
     if (config < -1 || config >= kNumSpmmConfigs) return MC_EINVAL_ARG;
     // a batched launch fills the GPU with (row, tile) x batch workgroups
-    int cfg = config >= 0 ? config : default_config(rhs_bits, n, (long long)m_vec * batch);
+    const int rows = out16 ? 32 : mfma_rows(lhs_bits, rhs_bits, sign == MC_SIGNED, vec_length);
+    int cfg = config >= 0 ? config : default_config(rhs_bits, n, (long long)m_vec * batch, rows);
     if (!config_supported(cfg, rhs_bits)) return MC_EUNSUPPORTED;
     if (batch > 1 && kSpmmConfigs[cfg].kind == 1) return MC_EUNSUPPORTED;   // B-stationary: one matrix
     if (kSpmmConfigs[cfg].kind == 1 && !stationary_fits(cfg, n, k)) {
         if (config >= 0) return MC_EINVAL_SHAPE;
         cfg = 7;   // the gather kernel takes any k
     }
-    if ((n / cpd) % kSpmmConfigs[cfg].lane_dwords != 0) {
-        if (config >= 0) return MC_EINVAL_SHAPE;
-        cfg = 4;   // one dword per lane fits every n
-    }
+    // an explicit tile's lanes divide a row; the default's last lane may
+    // repeat columns of its neighbour
+    if (config >= 0 && (n / cpd) % kSpmmConfigs[cfg].lane_dwords != 0) return MC_EINVAL_SHAPE;
 
     SpmmArgs a{};
     a.m_vec = m_vec;

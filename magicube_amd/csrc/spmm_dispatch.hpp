@@ -10,15 +10,16 @@
 namespace mc {
 
 // Tile configurations {lane_dwords, tiles_per_block, split_k, depth, kind,
-// waves_per_simd}: 0-7 and 12-23 gather kernel (four dwords per lane: 8- and
+// waves_per_simd}: 0-7 and 12-25 gather kernel (four dwords per lane: 8- and
 // 16-bit B); 8-11 B-stationary kernel (8-bit B), for which the fields are {B dwords per slice row, waves per workgroup,
 // vector rows per workgroup, prefetch depth}.  waves_per_simd > 1 makes the
 // register allocation fit that many waves per SIMD.  13 and 14 are config 7
 // with one and two k-blocks of gathers in flight per wave instead of three
 // (the software-pipelining ablation).  15-23 vary the waves per row (1, 2,
-// 4, 8), the split of a row's k-blocks over waves and the depth; the defaults
-// (15, 16, 17, 20, 22) come from them.
-constexpr int kNumSpmmConfigs = 24;
+// 4, 8), the split of a row's k-blocks over waves and the depth; 24 and 25 load
+// 16 bytes per lane with one k-block in flight.  The defaults (13, 15, 16, 17,
+// 20, 22, 24) come from them.
+constexpr int kNumSpmmConfigs = 26;
 constexpr mc_tile_config kSpmmConfigs[kNumSpmmConfigs] = {
     {2, 4, 1, 2, 0, 0}, {2, 4, 2, 2, 0, 0}, {4, 2, 2, 2, 0, 0}, {4, 2, 4, 2, 0, 0},
     {1, 4, 2, 3, 0, 0}, {2, 2, 2, 2, 0, 0}, {4, 1, 4, 2, 0, 0}, {1, 8, 1, 3, 0, 0},
@@ -26,7 +27,7 @@ constexpr mc_tile_config kSpmmConfigs[kNumSpmmConfigs] = {
     {1, 4, 1, 2, 0, 6}, {1, 8, 1, 1, 0, 0}, {1, 8, 1, 2, 0, 0},
     {1, 1, 1, 1, 0, 0}, {1, 2, 1, 1, 0, 0}, {1, 4, 1, 1, 0, 0}, {1, 2, 1, 2, 0, 0},
     {1, 4, 1, 3, 0, 0}, {1, 4, 2, 1, 0, 0}, {1, 8, 2, 1, 0, 0}, {1, 2, 2, 1, 0, 0},
-    {1, 4, 2, 2, 0, 0},
+    {1, 4, 2, 2, 0, 0}, {4, 2, 1, 1, 0, 0}, {4, 8, 1, 1, 0, 0},
 };
 
 // Whether a B-stationary config fits the shape (slice width divides n, the
@@ -40,7 +41,8 @@ inline bool stationary_fits(int cfg, int n, int k) {
 template <int V, int AB, int BB, bool SGN, int LW, int TPB, int SK, int D, int WPS = 1, bool LAYER = false>
 mc_status spmm_launch_one(SpmmArgs a, hipStream_t stream) {
     constexpr int TILE_N = 16 * LW * (32 / BB);
-    if ((a.n / (32 / BB)) % LW != 0) return MC_EUNSUPPORTED;
+    // a lane's dwords lie in one row; rows are stored four columns at a time
+    if (LW > 1 && (a.n / (32 / BB) < LW || a.n % 4 != 0)) return MC_EUNSUPPORTED;
     a.tiles_n = (a.n + TILE_N - 1) / TILE_N;
     const int groups = (a.tiles_n + TPB - 1) / TPB;
     const long long blocks = (long long)a.m_vec * groups;
@@ -92,6 +94,12 @@ mc_status spmm_launch_cfg(int cfg, const SpmmArgs &a, hipStream_t s) {
     case 21: return spmm_launch_one<V, AB, BB, SGN, 1, 8, 2, 1>(a, s);
     case 22: return spmm_launch_one<V, AB, BB, SGN, 1, 2, 2, 1>(a, s);
     case 23: return spmm_launch_one<V, AB, BB, SGN, 1, 4, 2, 2>(a, s);
+    case 24:
+        if constexpr (BB != 4) return spmm_launch_one<V, AB, BB, SGN, 4, 2, 1, 1>(a, s);
+        else return MC_EUNSUPPORTED;
+    case 25:
+        if constexpr (BB != 4) return spmm_launch_one<V, AB, BB, SGN, 4, 8, 1, 1>(a, s);
+        else return MC_EUNSUPPORTED;
     default: return MC_EINVAL_ARG;
     }
 }

@@ -330,8 +330,11 @@ __global__ __launch_bounds__(64 * TPB * SPLITK) __attribute__((amdgpu_waves_per_
     const int aend = start + ((end - start + MMA_K - 1) / MMA_K) * MMA_K;
 
     const int n_dw = args.n / CPD;                        // dwords per B row
-    const int col_dw = tile * (TILE_N / CPD) + r * LW;    // first dword of this lane
-    const bool col_ok = (tile < args.tiles_n) && (col_dw < n_dw);
+    // first dword of this lane; where a row's last LW dwords straddle its end
+    // the lane starts earlier and repeats columns of its neighbour
+    const int own_dw = tile * (TILE_N / CPD) + r * LW;
+    const bool col_ok = (tile < args.tiles_n) && (own_dw < n_dw);
+    const int col_dw = LW == 1 ? own_dw : min(own_dw, n_dw - LW);
     const u32 row_stride = (u32)n_dw * 4u;
     // lanes past the last column add kOobAdd: real rows then read out of range
     const u32 coff = col_ok ? (u32)col_dw * 4u : kOobAdd;
@@ -427,6 +430,7 @@ __global__ __launch_bounds__(64 * TPB * SPLITK) __attribute__((amdgpu_waves_per_
                 *reinterpret_cast<v4i *>(s_a + 16 * i) = buf_load_b128(ra, a_base + 16u * (u32)i);
         }
         __syncthreads();
+        if (tile >= args.tiles_n) continue;     // no columns: this wave only helps staging
 
         // Branch-free issue: the LDS block index is clamped into the chunk and
         // validity rides on one additive offset (B is < 1 GiB, so adding
@@ -512,35 +516,39 @@ __global__ __launch_bounds__(64 * TPB * SPLITK) __attribute__((amdgpu_waves_per_
         }
     }
 
-    // sums mod 2^32 in unsigned arithmetic
-    u32 comb[NMMA][HOME];
+    // accumulator group j, home row i: planes recombined mod 2^32
+    auto combined = [&](int j, int i) {
+        u32 vsum = 0;
 #pragma unroll
-    for (int j = 0; j < NMMA; ++j)
-#pragma unroll
-        for (int i = 0; i < HOME; ++i) {
-            u32 vsum = 0;
-#pragma unroll
-            for (int p = 0; p < P; ++p) {
-                int t, dg, di;
-                if constexpr (V == 8) { t = p / 2; dg = 2 * (p % 2); di = 0; }
-                else if constexpr (V == 4) { t = p / 4; dg = p % 4; di = 0; }
-                else { t = p / 8; dg = (p % 8) / 2; di = 2 * (p % 2); }
-                int x = acc[t][j][i + di];
-                if (dg != 0) x = lane_down(x, 16 * dg);
-                vsum += (u32)T::weight(p) * (u32)x;
-            }
-            comb[j][i] = vsum;
+        for (int p = 0; p < P; ++p) {
+            int t, dg, di;
+            if constexpr (V == 8) { t = p / 2; dg = 2 * (p % 2); di = 0; }
+            else if constexpr (V == 4) { t = p / 4; dg = p % 4; di = 0; }
+            else { t = p / 8; dg = (p % 8) / 2; di = 2 * (p % 2); }
+            int x = acc[t][j][i + di];
+            if (dg != 0) x = lane_down(x, 16 * dg);
+            vsum += (u32)T::weight(p) * (u32)x;
         }
-    int res[NCOL][HOME];
+        return vsum;
+    };
+    // output column c of home row i
+    auto value = [&](int c, int i) {
+        u32 x;
+        if constexpr (BB == 16) x = (combined(2 * c + 1, i) << 8) + combined(2 * c, i);
+        else x = combined(c, i);
+        return (int)(x + (u32)OB * (u32)rs_home[i]);
+    };
+    // whole rows at once where they are reduced or stored directly; the LDS
+    // store below takes its two rows at a time (with several planes and 16
+    // columns per lane the whole set does not fit the registers)
+    constexpr bool kRowPairs = NCOL > 4 && SPLITK == 1 && !LAYER;
+    int res[kRowPairs ? 1 : NCOL][HOME];
+    if constexpr (!kRowPairs) {
 #pragma unroll
-    for (int c = 0; c < NCOL; ++c)
+        for (int c = 0; c < NCOL; ++c)
 #pragma unroll
-        for (int i = 0; i < HOME; ++i) {
-            u32 x;
-            if constexpr (BB == 16) x = (comb[2 * c + 1][i] << 8) + comb[2 * c][i];
-            else x = comb[c][i];
-            res[c][i] = (int)(x + (u32)OB * (u32)rs_home[i]);
-        }
+            for (int i = 0; i < HOME; ++i) res[c][i] = value(c, i);
+    }
 
     const bool home = g < (V + 3) / 4;
     if constexpr (SPLITK > 1) {
@@ -569,8 +577,8 @@ __global__ __launch_bounds__(64 * TPB * SPLITK) __attribute__((amdgpu_waves_per_
         }
     }
 
-    if (!home || !col_ok) return;
     if constexpr (LAYER) {
+        if (!home || !col_ok) return;
         // read next by the output projection: plain stores
         __half *const out16 = args.out16 + bz * args.out_stride;
 #pragma unroll
@@ -591,17 +599,69 @@ __global__ __launch_bounds__(64 * TPB * SPLITK) __attribute__((amdgpu_waves_per_
         }
         return;
     }
+    if constexpr (NCOL > 4) {
+        // A lane's columns span 32 bytes or more, so its 16-byte stores would
+        // leave every line to several instructions (non-temporal partial
+        // lines: 64 us against 33 for plain stores and 20 for whole lines,
+        // 4096 x 4096 x 4096, 98 % sparse).  Two rows at a time pass through a
+        // per-wave LDS tile, from which the wave stores them contiguously.
+        __shared__ __attribute__((aligned(16))) int s_out[TPB][2 * TILE_N];
+        if (tile >= args.tiles_n) return;
+        int *const st = s_out[tile_local];
+        int *const tile0 = out + (size_t)m * V * (size_t)args.n + (size_t)tile * TILE_N;
+        const int cols = min(TILE_N, args.n - tile * TILE_N);       // a multiple of 4
+#pragma unroll
+        for (int p = 0; p < V / 2; ++p) {
+            // V = 8: rows p and 4 + p; else rows 2p and 2p + 1
+            const int at = col_dw * CPD - tile * TILE_N;        // < 0: columns of the tile before
+#pragma unroll
+            for (int h = 0; h < (V == 8 ? 1 : 2); ++h) {
+                const int i = V == 8 ? p : 2 * p + h;
+                int *o = st + (V == 8 ? g : h) * TILE_N + at;
+#pragma unroll
+                for (int c0 = 0; c0 < NCOL; c0 += 4) {
+                    int x[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if constexpr (kRowPairs) x[e] = value(c0 + e, i);     // every lane (lane moves)
+                        else x[e] = res[c0 + e][i];
+                    }
+                    if (!home || !col_ok) continue;
+                    if constexpr (CPD < 4) {
+                        if (LW == 1 || at + c0 >= 0) *reinterpret_cast<v2i *>(o + c0) = v2i{x[0], x[1]};
+                        if (LW == 1 || at + c0 + 2 >= 0) *reinterpret_cast<v2i *>(o + c0 + 2) = v2i{x[2], x[3]};
+                    } else if (LW == 1 || at + c0 >= 0) {
+                        *reinterpret_cast<v4i *>(o + c0) = v4i{x[0], x[1], x[2], x[3]};
+                    }
+                }
+            }
+            // the tile is the wave's own and its LDS operations complete in order
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int k = 0; k < TILE_N / 128; ++k) {
+                const int e = (64 * k + lane) * 4, h = e / TILE_N, col = e % TILE_N;
+                const int row = V == 8 ? p + 4 * h : 2 * p + h;
+                const v4i o = *reinterpret_cast<const v4i *>(st + e);
+                if (col < cols)
+                    __builtin_nontemporal_store(o, reinterpret_cast<v4i *>(tile0 + (size_t)row * (size_t)args.n + col));
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        return;
+    }
+    if (!home || !col_ok) return;
     // lane r owns dwords [col_dw, col_dw + LW): NCOL consecutive columns
 #pragma unroll
     for (int i = 0; i < HOME; ++i) {
         const int v = 4 * g + i;
         int *orow = out + (size_t)(m * V + v) * (size_t)args.n + (size_t)col_dw * CPD;
-        if constexpr (NCOL % 4 == 0) {
-#pragma unroll
-            for (int c4 = 0; c4 < NCOL; c4 += 4) {
-                v4i o = v4i{res[c4][i], res[c4 + 1][i], res[c4 + 2][i], res[c4 + 3][i]};
-                __builtin_nontemporal_store(o, reinterpret_cast<v4i *>(orow + c4));
-            }
+        if constexpr (NCOL == 4) {
+            v4i o = v4i{res[0][i], res[1][i], res[2][i], res[3][i]};
+            __builtin_nontemporal_store(o, reinterpret_cast<v4i *>(orow));
         } else {
 #pragma unroll
             for (int c2 = 0; c2 < NCOL; c2 += 2) {
