@@ -7,10 +7,13 @@ namespace {
 
 constexpr int kMaxWaves = 8;   // waves per row
 
-// Waves per row W and tiles per group T.  Under 1024 rows (times the batch) a
+// Waves per row W and tiles per group T.  Under 768 rows (times the batch) a
 // launch is one round of workgroups, so a row is spread over more waves and,
 // at K <= 128, single tiles; from there on fewer waves with longer pipelines
-// keep more rows resident.  Measured on MI355X, us (rows x N, K, sparsity):
+// keep more rows resident (819 rows x 5463, K = 448, 93 % sparse, operands not
+// in the caches: W4 18.9 us, W8 23.3).  At K = 256 two tiles' gathers take the
+// registers of a wave more per SIMD: T1 (1000 rows x 8000, 80 % sparse: 28.2
+// against 30.5 us; 819 rows, K = 192: 10.9 against 12.3).  Measured on MI355X, us (rows x N, K, sparsity):
 //                            W8 T1   W8 T2   W4 T1   W4 T2   W2 T2   W16 T1
 //   512 x 4096, 64, 0.9        4.9     5.0     5.7     5.6     7.3     5.6
 //   512 x 4096, 128, 0.9       5.4     5.6     6.1     6.1     7.8     6.6
@@ -30,14 +33,16 @@ mc_status sddmm_launch_tiles(const SddmmArgs &a, int waves, int batch, hipStream
 
 template <int V, int BITS, bool SGN, int NKC, int OUT>
 mc_status sddmm_launch(const SddmmArgs &a, int batch, hipStream_t s) {
-    const bool one_round = (long long)a.m_vec * batch < 1024;
+    const bool one_round = (long long)a.m_vec * batch < 768;
     const int waves = one_round ? 8 : 4;
-    if constexpr (BITS == 16) {
+    if constexpr (BITS == 16 || NKC == 4) {
         return sddmm_launch_tiles<V, BITS, SGN, NKC, 1, OUT>(a, waves, batch, s);
-    } else if constexpr (NKC <= 2) {
-        if (one_round) return sddmm_launch_tiles<V, BITS, SGN, NKC, 1, OUT>(a, waves, batch, s);
+    } else {
+        if constexpr (NKC <= 2) {
+            if (one_round) return sddmm_launch_tiles<V, BITS, SGN, NKC, 1, OUT>(a, waves, batch, s);
+        }
+        return sddmm_launch_tiles<V, BITS, SGN, NKC, 2, OUT>(a, waves, batch, s);
     }
-    if constexpr (BITS != 16) return sddmm_launch_tiles<V, BITS, SGN, NKC, 2, OUT>(a, waves, batch, s);
 }
 
 template <int V, int BITS, bool SGN, int OUT>
