@@ -69,6 +69,10 @@ class DeviceMask:
     row_offsets: torch.Tensor
     col_indices: torch.Tensor
     row_indices: torch.Tensor
+    # every output slot belongs to a row's [start, roundup8(end)): a product
+    # writes the whole output, which then needs no zero fill (as much as a
+    # third of the time of one: 5.5 of 17.5 us for 27 MB)
+    covered: bool = False
 
     @classmethod
     def upload(cls, csr: formats.VectorCSR, alignment: int = 8, device="cuda") -> "DeviceMask":
@@ -80,7 +84,10 @@ class DeviceMask:
             a = np.ascontiguousarray(a) if a.size else np.full(16, fill, np.int32)
             return torch.from_numpy(a).to(device)
 
-        return cls(csr.m_vec, csr.k, csr.V, an, pairs, cols, t(pairs, 0), t(cols, -1), t(order, 0))
+        # rows on 8 slots leave no gap, unless the arrays only hold the
+        # placeholders of an empty mask
+        return cls(csr.m_vec, csr.k, csr.V, an, pairs, cols, t(pairs, 0), t(cols, -1), t(order, 0),
+                   covered=alignment == 8 and cols.size == an > 0)
 
     def output_size(self) -> int:
         """int32 values the launch may write: the padded slot array rounded up to 8, times V."""
@@ -89,7 +96,8 @@ class DeviceMask:
     def sddmm(self, bits: int, lhs: torch.Tensor, rhs: torch.Tensor, k: int, out: torch.Tensor | None = None,
               sign: int = SIGNED, layout: int = OUT_REFERENCE, stream=None) -> torch.Tensor:
         if out is None:
-            out = torch.zeros(self.output_size(), dtype=torch.int32, device=lhs.device)
+            make = torch.empty if self.covered else torch.zeros
+            out = make(self.output_size(), dtype=torch.int32, device=lhs.device)
         wmma_sddmm(bits, self.m_vec, k, self.n, self.row_indices, self.row_offsets, self.col_indices, lhs, rhs,
                    out, self.V, sign, layout, stream)
         return out

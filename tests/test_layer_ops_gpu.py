@@ -143,3 +143,28 @@ def test_quantize_matches_the_restatement(bits, rows):
         exp = oatt.quantize_ref(t.contiguous().cpu().numpy(), 30.0, bits, 0)
         lanes = formats.unpack_lanes(got.cpu().numpy().view(np.uint8), bits, exp.size, signed=True)
         assert np.array_equal(lanes.reshape(exp.shape), exp)
+
+
+@pytest.mark.parametrize("alignment", [8, 16])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_sddmm_output_has_no_stale_slots(alignment, layout):
+    """A product into memory full of another value leaves 0 in every padding slot."""
+    from magicube_amd import sddmm
+    rng = np.random.default_rng(alignment)
+    ro = np.concatenate([[0], np.cumsum(COUNTS)]).astype(np.int32)
+    cols = np.concatenate([np.sort(rng.permutation(KEYS)[:c]) for c in COUNTS]).astype(np.int32)
+    for V, counts in ((8, COUNTS), (2, COUNTS), (4, (0, 0))):
+        csr = formats.VectorCSR(len(counts), KEYS, V, ro if counts is COUNTS else np.zeros(3, np.int32),
+                                cols if counts is COUNTS else cols[:0])
+        mask = sddmm.DeviceMask.upload(csr, alignment)
+        lhs = rng.integers(-128, 128, size=(len(counts) * V, 64))
+        rhs = rng.integers(-128, 128, size=(KEYS, 64))
+        junk = torch.full((mask.output_size(),), 9, dtype=torch.int32, device="cuda")
+        del junk        # the caching allocator hands this block to the output
+        out = mask.sddmm(8, packed(lhs, 8), packed(rhs, 8), 64, layout=layout).cpu().numpy()
+        slots = out.reshape(-1, V, 8).transpose(0, 2, 1).reshape(-1, V) if layout == 0 else out.reshape(-1, V)
+        exp = np.zeros_like(slots)
+        for i in range(len(counts)):
+            s, e = int(mask.pairs[2 * i]), int(mask.pairs[2 * i + 1])
+            exp[s:e] = rhs[mask.cols[s:e]] @ lhs[i * V:(i + 1) * V].T
+        assert np.array_equal(slots, exp)
