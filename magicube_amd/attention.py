@@ -445,9 +445,8 @@ class AttentionBatch:
         (stream if stream is not None else torch.cuda.current_stream()).wait_event(self._ready)
 
     # -- fused path ---------------------------------------------------------
-    def quantize(self, stream=None) -> None:
-        self._wait_ready(stream)
-        lib, st = _lib.lib(), _stream(stream)
+    def _launch_quantize(self, st: int) -> None:
+        lib = _lib.lib()
         n = len(self.mats)
         if self.all_jobs is not None:
             _lib.check(lib.mc_attn_quantize_batched(_dptr(self.all_jobs), self.n_first + n, self.qk_bits,
@@ -458,16 +457,25 @@ class AttentionBatch:
         _lib.check(lib.mc_attn_quantize_batched(_dptr(self.v_jobs), n, self.v_bits, self.v_rounding,
                                                 self.max_count, st), "mc_attn_quantize_batched")
 
+    def _launch_attend(self, st: int, grid_waves: int) -> None:
+        _lib.check(_lib.lib().mc_attn_forward(_dptr(self.desc), _dptr(self.items), self.n_items, self.qk_bits,
+                                              self.v_bits, self.V, self.p_scale, self.p_mode, grid_waves,
+                                              int(self.debug), st), "mc_attn_forward")
+
+    def quantize(self, stream=None) -> None:
+        self._wait_ready(stream)
+        self._launch_quantize(_stream(stream))
+
     def attend(self, stream=None, grid_waves: int = DEFAULT_GRID_WAVES) -> None:
         self._wait_ready(stream)
-        _lib.check(_lib.lib().mc_attn_forward(_dptr(self.desc), _dptr(self.items), self.n_items, self.qk_bits,
-                                              self.v_bits, self.V, self.p_scale, self.p_mode, grid_waves, int(self.debug),
-                                              _stream(stream)),
-                   "mc_attn_forward")
+        self._launch_attend(_stream(stream), grid_waves)
 
     def forward(self, stream=None, grid_waves: int = DEFAULT_GRID_WAVES) -> list[torch.Tensor]:
-        self.quantize(stream)
-        self.attend(stream, grid_waves)
+        """:meth:`quantize` then :meth:`attend`, on one look at the stream."""
+        self._wait_ready(stream)
+        st = _stream(stream)
+        self._launch_quantize(st)
+        self._launch_attend(st, grid_waves)
         return [d.o for d in self.mats]
 
     def capture(self, stream: torch.cuda.Stream, grid_waves: int = DEFAULT_GRID_WAVES) -> torch.cuda.CUDAGraph:

@@ -65,6 +65,7 @@ from torch import nn
 from . import _lib, formats
 from .attention import (HEAD_DIM, P_REFERENCE, P_REFERENCE_4BIT, ROUND_TRUNC, AttentionBatch, AttentionMatrix,
                         ResidentMask)
+from .spmm import current_stream_handle
 
 # plans (buffers, quantized operands, descriptors) kept per module, least
 # recently used dropped first
@@ -339,7 +340,7 @@ class FusedLayerNorm(nn.LayerNorm):
         st = _lib.lib().mc_layernorm_f16(x.numel() // x.shape[-1], x.shape[-1], x.data_ptr(),
                                          None if residual is None else residual.data_ptr(),
                                          None if w is None else w.data_ptr(), None if b is None else b.data_ptr(),
-                                         float(self.eps), out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+                                         float(self.eps), out.data_ptr(), current_stream_handle())
         if st:
             _lib.check(st, "mc_layernorm_f16")
         return out

@@ -43,17 +43,15 @@ import torch
 
 from . import _lib
 from .attention import bquantization as _bquantization
+from .spmm import current_stream_handle
 
 
 def _ptr(t):
-    import ctypes
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _stream_handle(stream):
-    import ctypes
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    return stream.cuda_stream if stream is not None else current_stream_handle()
 
 
 def _on(stream):
