@@ -32,9 +32,38 @@
 // order.
 #pragma once
 
+#include <hip/hip_fp16.h>
+
 #include "mc_device.hpp"
+#include "mc_internal.hpp"
 
 namespace mc {
+
+// Device view of mc_attn_matrix (same member order and types).
+struct AttnMatrix {
+    int L;
+    int m_vec;
+    const int *row_offsets;
+    const int *col_indices;
+    const unsigned char *q;
+    const unsigned char *k;
+    const unsigned char *v;
+    float alpha;
+    float o_scale;
+    float *o;
+    int *o_int;
+    unsigned char *p_out;
+    int *s_out;
+    __half *o16;
+    int o16_stride;
+    int o16_pad;
+    const __half *q16;
+    int q16_stride;
+    float q_scale;
+    int q_rounding;
+    int q_pad;
+};
+static_assert(sizeof(AttnMatrix) == sizeof(mc_attn_matrix), "descriptor layout");
 
 constexpr int kHeadDim = 64;
 

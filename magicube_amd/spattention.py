@@ -143,8 +143,8 @@ def _padded_mask(base: ResidentMask, base_cols: np.ndarray, drop: np.ndarray, de
 class _Plan:
     """Per (shape, mask, padding, precision) state of SpMultiheadAttention.
 
-    The in-projection writes ``qkv`` ([L][batch][3 * E] fp16); the quantize
-    launch reads each (sample, head)'s [L][64] slices of it in place, and the
+    The in-projection writes ``qkv`` ([L][batch][3 * E] fp16; see
+    :meth:`project`); the quantize launch reads each (sample, head)'s [L][64] slices of it in place, and the
     fused kernel writes each head's output as fp16 straight into ``o``
     ([L][batch][E], the output projection's input), so no permute copies run
     between the projections and the attention kernels.  ``masks`` holds one
@@ -177,6 +177,29 @@ class _Plan:
                               scales=[(SCALE_QKV, SCALE_QKV, SCALE_QKV)] * n_mat, rounding=ROUND_TRUNC,
                               device=self.device, outputs=outs, v_range4=self.rhs_pre == 4, debug=debug)
 
+    def project(self, x2: torch.Tensor, w: torch.Tensor, b) -> bool:
+        """The in-projection of x2 [L * batch][E] with K and V quantized as it
+        stores them (``mc_attn_in_projection_f16``): Q to ``qkv`` in fp16, K
+        and V to the batch's operands alone (their columns of ``qkv`` are left
+        as they were).  False, with nothing done, where the launch does not
+        apply.
+
+        It runs from 128 tiles of 128 x 128 on (half the CUs; below, the
+        library's product and a quantize launch are a few microseconds, bound
+        by the host) and up to E = 256: 32768 rows of E = 256 took 28 us and
+        the quantize launch 12 more, this launch 20 less than both.  At E = 512 the library's own product is a quarter
+        faster than this one, which cancels what the quantize launch took."""
+        rows, E = self.L * self.bsz, self.heads * HEAD_DIM
+        if (E % 128 or E > 256 or self.bsz * self.heads > 256 or -(-rows // 128) * (3 * E // 128) < 128
+                or not self.batch.fuse_q or not _vector_operands(x2, w, b, self.qkv)):
+            return False
+        self.batch._wait_ready(None)
+        _lib.check(_lib.lib().mc_attn_in_projection_f16(
+            self.L, self.bsz, self.heads, x2.data_ptr(), w.data_ptr(), None if b is None else b.data_ptr(), SCALE_QKV,
+            self.rhs_pre, int(self.rhs_pre == 4), self.batch.desc.data_ptr(), self.qkv.data_ptr(),
+            current_stream_handle()), "mc_attn_in_projection_f16")
+        return True
+
     def forward_with_weights(self) -> torch.Tensor:
         """Runs the layer through the kernel that also writes P and returns
         the head-averaged weights P / 32 as [batch, L, L] (float32)."""
@@ -203,6 +226,17 @@ class _Plan:
                 acc += mats[b * self.heads + h].p_out[p_idx].to(torch.int8).float()
             w[b].index_put_((r_idx, cols), acc / (SCALE_SFMX * self.heads))
         return w
+
+
+def _vector_operands(*ts) -> bool:
+    """fp16 operands (None allowed) a HIP launch on the current device reads
+    in 16-byte pieces, none of which needs a gradient."""
+    grad, dev = torch.is_grad_enabled(), torch.cuda.current_device()
+    for t in ts:
+        if t is not None and (not t.is_cuda or t.dtype != torch.float16 or t.get_device() != dev
+                              or not t.is_contiguous() or t.data_ptr() % 16 or (grad and t.requires_grad)):
+            return False
+    return True
 
 
 def _key_tensors(*ts):
@@ -282,9 +316,13 @@ class SpMultiheadAttention(nn.MultiheadAttention):
             raise NotImplementedError("the quantized path takes fp16 activations")
         w, b = self.in_proj_weight, self.in_proj_bias
         qkv2 = plan.qkv.view(L * bsz, 3 * E)
+        quantized = False
         if query is key and key is value:
             x2 = query.reshape(L * bsz, E)
-            if b is None:
+            quantized = not need_weights and plan.project(x2, w, b)
+            if quantized:
+                pass
+            elif b is None:
                 torch.mm(x2, w.t(), out=qkv2)
             else:
                 torch.addmm(b, x2, w.t(), out=qkv2)
@@ -295,7 +333,10 @@ class SpMultiheadAttention(nn.MultiheadAttention):
         if need_weights:
             weights = plan.forward_with_weights().to(query.dtype)
         else:
-            plan.batch.forward()
+            if quantized:
+                plan.batch.attend()
+            else:
+                plan.batch.forward()
             weights = None
         return F.linear(plan.o, self.out_proj.weight, self.out_proj.bias), weights
 
