@@ -376,16 +376,10 @@ mc_status mc_attn_forward(const mc_attn_matrix *matrices, const int *items, int 
 mc_status mc_layernorm_f16(long long rows, int cols, const void *x, const void *residual, const void *weight,
                            const void *bias, float eps, void *out, hipStream_t stream);
 
-/* Linear layer on fp16 rows, accumulated in fp32:
- *   out = half(x w^T + bias), or half(out + residual) when residual is non-null
- * x [rows][k], w [n][k], bias [n] (may be null), residual and out [rows][n],
- * all 16-byte aligned; n a multiple of 128, k of 64. */
-mc_status mc_linear_f16(long long rows, int n, int k, const void *x, const void *w, const void *bias,
-                        const void *residual, void *out, hipStream_t stream);
-
 /* The attention module's in-projection: qkv = half(x w^T + bias) over rows
  * l * samples + b of heads * 64 columns (w [3 * heads * 64][heads * 64], the
- * Q, K and V rows in turn; heads even).  Q is stored to qkv ([rows][3 * heads
+ * Q, K and V rows in turn; heads even, 3 * heads * 64 <= 4096, samples *
+ * heads <= 256; x, w, bias and qkv 16-byte aligned).  Q is stored to qkv ([rows][3 * heads
  * * 64]; its K and V columns are left alone); K and V are quantized as
  * mc_attn_quantize_batched does, with MC_ROUND_TRUNC and `scale`, into the k
  * and v buffers of the device descriptors matrices[b * heads + h]: K at

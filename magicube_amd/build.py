@@ -42,7 +42,7 @@ LIB_SOURCES = [
     "spmm_layer.hip",
     "gaps.hip",
 ]
-OPTIONAL_SOURCES = ["sddmm.hip", "attention.hip", "layernorm.hip", "linear.hip"]
+OPTIONAL_SOURCES = ["sddmm.hip", "attention.hip", "layernorm.hip", "in_projection.hip"]
 # Vendor-library comparators (rocSPARSE, hipBLASLt): a library of their own so
 # the product library carries no dependency on them.
 VENDOR_LIB = os.path.join(HERE, "libmagicube_vendor.so")

@@ -1,8 +1,7 @@
-// fp16 linear layers of the encoder on many rows:
-//   y = half(x w^T + bias), or half(y + residual)     (accumulated in fp32)
-// and the attention module's in-projection, which quantizes K and V as it
-// stores them.  The reference leaves these products to torch
-// (end2end_eval/sparse_transformer_magicube/end_to_end.py:47-89, spattention.py).
+// The attention module's in-projection y = half(x w^T + bias) on many rows,
+// accumulated in fp32, which quantizes K and V as it stores them.  The
+// reference leaves the product to torch and quantizes in a launch of its own
+// (end2end_eval/sparse_transformer_magicube/spattention.py).
 #include <hip/hip_fp16.h>
 
 #include "attention_common.hpp"
@@ -17,15 +16,14 @@ constexpr int kTileM = 128, kTileN = 128, kTileK = 64;     // rows of x, columns
 constexpr int kMaxCols = 4096, kMaxMats = 256;             // bias columns and (sample, head) matrices held in LDS
 constexpr int kWave = 64;                                  // a wave's tile: 64 rows x 64 columns
 
-struct LinearArgs {
+struct ProjectionArgs {
     long long rows;
     int n, k;
     const __half *x;            // [rows][k]
     const __half *w;            // [n][k]
     const __half *bias;         // [n] or null
-    const __half *res;          // [rows][n] or null
-    __half *out;                // [rows][n]
-    // in-projection: row l * samples + b, columns [Q | K | V] of heads x 64
+    __half *out;                // [rows][n]: its Q columns
+    // row l * samples + b, columns [Q | K | V] of heads x 64
     const AttnMatrix *mats;     // matrix b * heads + h
     int samples, heads;
     float scale;
@@ -39,7 +37,7 @@ __device__ __forceinline__ v4f mfma_f16(const v4i &a, const v4i &b, const v4f &c
 __device__ __forceinline__ __half2 as_half2(int x) { return *reinterpret_cast<const __half2 *>(&x); }
 __device__ __forceinline__ int as_int(const __half2 &x) { return *reinterpret_cast<const int *>(&x); }
 
-// KB: 0 stores y; 8 or 4 is the in-projection with that many bits per K value.
+// KB: bits per K value.
 //
 // y^T = w x^T on the matrix cores, so that a lane's accumulators are 16
 // consecutive columns of one row: the rows of w go to LDS in the order that
@@ -48,21 +46,24 @@ __device__ __forceinline__ int as_int(const __half2 &x) { return *reinterpret_ca
 // through LDS in 64-deep stages of 128-byte rows, whose 16-byte pieces are
 // xor-ed with the row (no bank conflicts for the writes or the MFMA reads).
 // Persistent workgroups, two per CU, walk (row block, column block) tiles:
-// the loads of the next two stages, of the next tile at a tile's end, are in
-// flight while a stage is multiplied or a tile stored.  An XCD takes whole row
+// the next stage's loads, of the next tile at a tile's end, are in flight
+// while a stage is multiplied or a tile stored.  An XCD takes whole row
 // blocks, so that x crosses HBM once and the column blocks read it from L2.
 //
-// 32768 rows, K = 256: N = 256 12 us (torch's product 20), N = 768 28 (28; with
-// the quantize launch it replaces 40); N = 1024 39 (31).  The in-projection
-// stores half of what the two launches moved: a batch-8 attention module of
-// L = 4096, E = 256 went from 126.6 to 107.0 us.
+// 32768 rows of 256 to 768 take 28 us with y stored whole, as torch's product
+// does, and the quantize launch that this replaces 12 more; a batch-8 attention
+// module of L = 4096, E = 256 went from 126.6 to 107.0 us.  MFMA, LDS and L1
+// are each busy about a quarter of the time (rows of 512 to 1536), without
+// bank conflicts.  Two stages' loads kept in flight over the barrier, the next
+// stage written to LDS under the products, and one tile per workgroup took
+// the same time or (the last) a fifth more.
 template <int KB>
-__global__ __launch_bounds__(256, 2) void linear_kernel(LinearArgs a, int mb, int nb) {
+__global__ __launch_bounds__(256, 2) void in_projection_kernel(ProjectionArgs a, int mb, int nb) {
     __shared__ v4i xs[2][kTileM * 8], ws[2][kTileN * 8];
     // bias and K / V buffers: from LDS, because a wait for a load at a tile's
     // end would also wait for the stages under way
     __shared__ __attribute__((aligned(16))) __half bs[kMaxCols];
-    __shared__ unsigned char *kv[KB ? 2 : 1][KB ? kMaxMats : 1];
+    __shared__ unsigned char *kv[2][kMaxMats];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 15, g = lane >> 4;
     const int wm = (wave & 1) * kWave, wn = (wave >> 1) * kWave;
@@ -84,8 +85,7 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(LinearArgs a, int mb, in
         const int col = (r & 64) + 16 * ((r >> 2) & 3) + 4 * ((r >> 4) & 3) + (r & 3);
         wrow[i] = (u32)(col * a.k + piece * 8) * 2u;
     }
-    // past the walk's end the last stage is loaded again (and not used): a
-    // load behind a branch would make every wait drain the loads after it
+    // past the walk's end the last stage is loaded again (and not used)
     const auto load = [&](Stage &s) {
         const int rb = next_tile / nb;
         const long long m0 = (long long)(xcd + 8 * rb) * kTileM;
@@ -122,13 +122,10 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(LinearArgs a, int mb, in
         for (int j = 0; j < 4; ++j) acc[m][j] = v4f{0.f, 0.f, 0.f, 0.f};
     Stage ra, rb;                                                // stages it + 1 and it + 2 of the walk
     for (int i = tid; i < a.n; i += 256) bs[i] = a.bias ? a.bias[i] : __half(0.f);
-    if constexpr (KB != 0) {
-        for (int i = tid; i < a.samples * a.heads; i += 256) {
-            kv[0][i] = const_cast<unsigned char *>(a.mats[i].k);
-            kv[1][i] = const_cast<unsigned char *>(a.mats[i].v);
-        }
+    for (int i = tid; i < a.samples * a.heads; i += 256) {
+        kv[0][i] = const_cast<unsigned char *>(a.mats[i].k);
+        kv[1][i] = const_cast<unsigned char *>(a.mats[i].v);
     }
-    // in this order: each wait of the loop then leaves the younger stage's loads in flight
     load(ra);
     __builtin_amdgcn_sched_barrier(0);
     load(rb);
@@ -158,7 +155,7 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(LinearArgs a, int mb, in
             const int n0 = tile % nb * kTileN + wn;              // wave-uniform: one head's columns
             const v4i b0 = *reinterpret_cast<const v4i *>(bs + n0 + 16 * g),
                       b1 = *reinterpret_cast<const v4i *>(bs + n0 + 16 * g + 8);
-            const int head = n0 >> 6, part = KB ? head / a.heads : 0;
+            const int head = n0 >> 6, part = head / a.heads;
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 const long long row = m0 + 16 * m + c;
@@ -172,14 +169,8 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(LinearArgs a, int mb, in
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[m][j] = v4f{0.f, 0.f, 0.f, 0.f};
                 if (row >= a.rows) continue;
-                if (KB == 0 || part == 0) {
+                if (part == 0) {
                     const size_t o = (size_t)row * a.n + n0 + 16 * g;
-                    if (KB == 0 && a.res) {
-                        const v4i r0 = *reinterpret_cast<const v4i *>(a.res + o),
-                                  r1 = *reinterpret_cast<const v4i *>(a.res + o + 8);
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) y[e] = __hadd2(y[e], as_half2(e < 4 ? r0[e & 3] : r1[e & 3]));
-                    }
                     *reinterpret_cast<v4i *>(a.out + o) = v4i{as_int(y[0]), as_int(y[1]), as_int(y[2]), as_int(y[3])};
                     *reinterpret_cast<v4i *>(a.out + o + 8) = v4i{as_int(y[4]), as_int(y[5]), as_int(y[6]), as_int(y[7])};
                 } else {
@@ -193,7 +184,7 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(LinearArgs a, int mb, in
                         q[e] = (u32)(int)fminf(fmaxf(f, lo), hi);
                     }
                     const int r32 = (int)row, l = r32 / a.samples, b = r32 - l * a.samples;
-                    unsigned char *o = kv[KB ? part - 1 : 0][KB ? b * a.heads + head - part * a.heads : 0];
+                    unsigned char *o = kv[part - 1][b * a.heads + head - part * a.heads];
                     if (KB == 4 && part == 1) {
                         u32 t[2] = {0, 0};
 #pragma unroll
@@ -225,22 +216,13 @@ __global__ __launch_bounds__(256, 2) void linear_kernel(LinearArgs a, int mb, in
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-template <int KB> mc_status linear_launch(const LinearArgs &a, hipStream_t stream) {
+template <int KB> mc_status in_projection_launch(const ProjectionArgs &a, hipStream_t stream) {
     const int mb = (int)((a.rows + kTileM - 1) / kTileM), nb = a.n / kTileN;
     const long long per_xcd = (long long)((mb + 7) / 8) * nb;
     if (per_xcd > 0x3FFFFFFF) return MC_EINVAL_SHAPE;
     const int step = per_xcd < 64 ? (int)per_xcd : 64;           // two workgroups on each of 32 CUs
-    hipLaunchKernelGGL((linear_kernel<KB>), dim3(8 * step), dim3(256), 0, stream, a, mb, nb);
+    hipLaunchKernelGGL((in_projection_kernel<KB>), dim3(8 * step), dim3(256), 0, stream, a, mb, nb);
     return check_launch();
-}
-
-mc_status linear_check(long long rows, int n, int k, const void *x, const void *w, const void *bias,
-                       const void *residual, const void *out) {
-    if (rows < 0 || rows >= (1LL << 30) || n <= 0 || n > kMaxCols || n % kTileN || k <= 0 || k % kTileK || k > 1 << 20) return MC_EINVAL_SHAPE;
-    if (rows == 0) return MC_OK;
-    if (!x || !w || !out) return MC_EINVAL_ARG;
-    if (!aligned16(x) || !aligned16(w) || !aligned16(bias) || !aligned16(residual) || !aligned16(out)) return MC_EINVAL_ARG;
-    return MC_OK;
 }
 
 }  // namespace
@@ -248,32 +230,18 @@ mc_status linear_check(long long rows, int n, int k, const void *x, const void *
 
 extern "C" {
 
-mc_status mc_linear_f16(long long rows, int n, int k, const void *x, const void *w, const void *bias,
-                        const void *residual, void *out, hipStream_t stream) {
-    const mc_status st = mc::linear_check(rows, n, k, x, w, bias, residual, out);
-    if (st != MC_OK || rows == 0) return st;
-    mc::LinearArgs a{};
-    a.rows = rows;
-    a.n = n;
-    a.k = k;
-    a.x = static_cast<const __half *>(x);
-    a.w = static_cast<const __half *>(w);
-    a.bias = static_cast<const __half *>(bias);
-    a.res = static_cast<const __half *>(residual);
-    a.out = static_cast<__half *>(out);
-    return mc::linear_launch<0>(a, stream);
-}
-
 mc_status mc_attn_in_projection_f16(int seq_len, int samples, int heads, const void *x, const void *w,
                                     const void *bias, float scale, int qk_bits, int v_range4,
                                     const mc_attn_matrix *matrices, void *qkv, hipStream_t stream) {
     if (qk_bits != 8 && qk_bits != 4) return MC_EUNSUPPORTED;
     if (seq_len < 0 || samples <= 0 || heads <= 0 || (long long)samples * heads > mc::kMaxMats) return MC_EINVAL_SHAPE;
     const int e = heads * 64;
-    const mc_status st = mc::linear_check((long long)seq_len * samples, 3 * e, e, x, w, bias, nullptr, qkv);
-    if (st != MC_OK || seq_len == 0) return st;
-    if (!matrices) return MC_EINVAL_ARG;
-    mc::LinearArgs a{};
+    if (e % mc::kTileK || 3 * e % mc::kTileN || 3 * e > mc::kMaxCols || (long long)seq_len * samples >= (1LL << 30))
+        return MC_EINVAL_SHAPE;
+    if (seq_len == 0) return MC_OK;
+    if (!x || !w || !qkv || !matrices) return MC_EINVAL_ARG;
+    if (!mc::aligned16(x) || !mc::aligned16(w) || !mc::aligned16(bias) || !mc::aligned16(qkv)) return MC_EINVAL_ARG;
+    mc::ProjectionArgs a{};
     a.rows = (long long)seq_len * samples;
     a.n = 3 * e;
     a.k = e;
@@ -286,7 +254,7 @@ mc_status mc_attn_in_projection_f16(int seq_len, int samples, int heads, const v
     a.heads = heads;
     a.scale = scale;
     a.v_range4 = v_range4;
-    return qk_bits == 8 ? mc::linear_launch<8>(a, stream) : mc::linear_launch<4>(a, stream);
+    return qk_bits == 8 ? mc::in_projection_launch<8>(a, stream) : mc::in_projection_launch<4>(a, stream);
 }
 
 }  // extern "C"

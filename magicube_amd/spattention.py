@@ -191,7 +191,8 @@ class _Plan:
         faster than this one, which cancels what the quantize launch took."""
         rows, E = self.L * self.bsz, self.heads * HEAD_DIM
         if (E % 128 or E > 256 or self.bsz * self.heads > 256 or -(-rows // 128) * (3 * E // 128) < 128
-                or not self.batch.fuse_q or not _vector_operands(x2, w, b, self.qkv)):
+                or not self.batch.fuse_q or not _vector_operands(x2, w, b, self.qkv) or tuple(x2.shape) != (rows, E)
+                or tuple(w.shape) != (3 * E, E) or (b is not None and tuple(b.shape) != (3 * E,))):
             return False
         self.batch._wait_ready(None)
         _lib.check(_lib.lib().mc_attn_in_projection_f16(
