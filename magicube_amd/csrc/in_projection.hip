@@ -54,9 +54,10 @@ __device__ __forceinline__ int as_int(const __half2 &x) { return *reinterpret_ca
 // does, and the quantize launch that this replaces 12 more; a batch-8 attention
 // module of L = 4096, E = 256 went from 126.6 to 107.0 us.  MFMA, LDS and L1
 // are each busy about a quarter of the time (rows of 512 to 1536), without
-// bank conflicts.  Two stages' loads kept in flight over the barrier, the next
-// stage written to LDS under the products, and one tile per workgroup took
-// the same time or (the last) a fifth more.
+// bank conflicts.  Not faster: two stages' loads kept in flight over the
+// barrier, the next stage written to LDS under the products, three workgroups
+// per CU with 32-deep stages, 256-row tiles; one and a half workgroups per CU
+// cost 6 us, one tile per workgroup 5.
 template <int KB>
 __global__ __launch_bounds__(256, 2) void in_projection_kernel(ProjectionArgs a, int mb, int nb) {
     __shared__ v4i xs[2][kTileM * 8], ws[2][kTileN * 8];
