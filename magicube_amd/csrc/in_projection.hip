@@ -50,8 +50,8 @@ __device__ __forceinline__ int as_int(const __half2 &x) { return *reinterpret_ca
 // while a stage is multiplied or a tile stored.  An XCD takes whole row
 // blocks, so that x crosses HBM once and the column blocks read it from L2.
 //
-// 32768 rows of 256 to 768 take 28 us with y stored whole, as torch's product
-// does, and the quantize launch that this replaces 12 more; a batch-8 attention
+// 32768 rows of 256 to 768 take 30 us (kernel trace), where torch's product and
+// the quantize launch took 27 and 12; a batch-8 attention
 // module of L = 4096, E = 256 went from 126.6 to 107.0 us.  MFMA, LDS and L1
 // are each busy about a quarter of the time (rows of 512 to 1536), without
 // bank conflicts.  Not faster: two stages' loads kept in flight over the

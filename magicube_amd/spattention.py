@@ -187,7 +187,8 @@ class _Plan:
         It runs from 128 tiles of 128 x 128 on (half the CUs; below, the
         library's product and a quantize launch are a few microseconds, bound
         by the host) and up to E = 256: 32768 rows of E = 256 took 28 us and
-        the quantize launch 12 more, this launch 20 less than both.  At E = 512 the library's own product is a quarter
+        the quantize launch 12 more; this launch takes 30, and a module
+        pass 20 less.  At E = 512 the library's own product is a quarter
         faster than this one, which cancels what the quantize launch took."""
         rows, E = self.L * self.bsz, self.heads * HEAD_DIM
         if (E % 128 or E > 256 or self.bsz * self.heads > 256 or -(-rows // 128) * (3 * E // 128) < 128
