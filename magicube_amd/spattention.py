@@ -61,6 +61,7 @@ import numpy as np
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.autograd import forward_ad
 
 from . import _lib, formats
 from .attention import (HEAD_DIM, P_REFERENCE, P_REFERENCE_4BIT, ROUND_TRUNC, AttentionBatch, AttentionMatrix,
@@ -232,7 +233,10 @@ class _Plan:
 
 def _vector_operands(*ts) -> bool:
     """fp16 operands (None allowed) a HIP launch on the current device reads
-    in 16-byte pieces, none of which needs a gradient."""
+    in 16-byte pieces, none of which needs a gradient.  Inside a forward-mode
+    AD level an operand may carry a tangent, which a launch would drop."""
+    if forward_ad._current_level >= 0:
+        return False
     grad, dev = torch.is_grad_enabled(), torch.cuda.current_device()
     for t in ts:
         if t is not None and (not t.is_cuda or t.dtype != torch.float16 or t.get_device() != dev
