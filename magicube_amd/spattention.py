@@ -356,13 +356,14 @@ class FusedLayerNorm(nn.LayerNorm):
 
     def _fast(self, x, residual) -> bool:
         """The HIP kernel's preconditions: fp16 operands on the current
-        device, contiguous, x and residual 8-byte aligned (four halves per
-        load), a supported width, and no operand that needs a gradient.
+        device, contiguous, x and residual 8-byte aligned (the launch's
+        loads), a supported width, and no operand that needs a gradient or
+        may carry a forward-mode tangent.
         Checked with cheap attribute reads: the encoder's eager forward is
         bound by host time."""
         n = self.normalized_shape[0] if len(self.normalized_shape) == 1 else 0
         if (n not in (256, 512, 1024) or not x.is_cuda or x.dtype != torch.float16 or x.shape[-1] != n
-                or not x.is_contiguous() or x.data_ptr() % 8):
+                or not x.is_contiguous() or x.data_ptr() % 8 or forward_ad._current_level >= 0):
             return False
         dev = x.get_device()
         if dev != torch.cuda.current_device():

@@ -2,6 +2,7 @@
 torch refuses a call or has a subclass handle it, so does the module."""
 import pytest
 import torch
+import torch.nn.functional as F
 from torch.autograd import forward_ad
 
 from magicube_amd import spattention
@@ -37,3 +38,15 @@ def test_forward_mode_tangents_are_refused(operand):
             setattr(mha, name, dual)
         with pytest.raises(NotImplementedError):
             mha(x, x, x, **args)
+
+
+@pytest.mark.parametrize("residual", [False, True])
+def test_layernorm_keeps_forward_mode_tangents(residual):
+    """torch's LayerNorm, which has them, runs inside a forward-mode level."""
+    ln = spattention.FusedLayerNorm(256).cuda().half()
+    x, t, r = (torch.randn(40, 256, device="cuda").half() for _ in range(3))
+    with torch.no_grad(), forward_ad.dual_level():
+        d = forward_ad.make_dual(x, t)
+        got = forward_ad.unpack_dual(ln(d, r) if residual else ln(d)).tangent
+        exp = forward_ad.unpack_dual(F.layer_norm(d + r if residual else d, (256,), ln.weight, ln.bias, ln.eps)).tangent
+    assert got is not None and torch.equal(got, exp)
