@@ -231,16 +231,21 @@ class _Plan:
         return w
 
 
+_PLAIN = (torch.Tensor, nn.Parameter)
+
+
 def _vector_operands(*ts) -> bool:
     """fp16 operands (None allowed) a HIP launch on the current device reads
     in 16-byte pieces, none of which needs a gradient.  Inside a forward-mode
-    AD level an operand may carry a tangent, which a launch would drop."""
+    AD level an operand may carry a tangent, which a launch would drop, and a
+    tensor subclass may hold its values elsewhere or watch torch's functions."""
     if forward_ad._current_level >= 0:
         return False
     grad, dev = torch.is_grad_enabled(), torch.cuda.current_device()
     for t in ts:
-        if t is not None and (not t.is_cuda or t.dtype != torch.float16 or t.get_device() != dev
-                              or not t.is_contiguous() or t.data_ptr() % 16 or (grad and t.requires_grad)):
+        if t is not None and (type(t) not in _PLAIN or not t.is_cuda or t.dtype != torch.float16
+                              or t.get_device() != dev or not t.is_contiguous() or t.data_ptr() % 16
+                              or (grad and t.requires_grad)):
             return False
     return True
 

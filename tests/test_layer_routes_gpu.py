@@ -50,3 +50,29 @@ def test_layernorm_keeps_forward_mode_tangents(residual):
         got = forward_ad.unpack_dual(ln(d, r) if residual else ln(d)).tangent
         exp = forward_ad.unpack_dual(F.layer_norm(d + r if residual else d, (256,), ln.weight, ln.bias, ln.eps)).tangent
     assert got is not None and torch.equal(got, exp)
+
+
+class Recorded(torch.Tensor):
+    """A tensor subclass that sees every torch function it passes through."""
+    seen = []
+
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        cls.seen.append(getattr(func, "__name__", str(func)))
+        return super().__torch_function__(func, types, args, kwargs or {})
+
+
+@pytest.mark.parametrize("operand", ["input", "weight"])
+def test_subclass_operands_reach_torch(operand):
+    """The in-projection of a tensor subclass is torch's addmm, which the subclass handles."""
+    mha, x, args = module()
+    if operand == "input":
+        x = x.as_subclass(Recorded)
+    else:
+        w = mha.in_proj_weight.detach().as_subclass(Recorded)
+        del mha.in_proj_weight
+        mha.in_proj_weight = w
+    Recorded.seen.clear()
+    with torch.no_grad():
+        mha(x, x, x, **args)
+    assert "addmm" in Recorded.seen
