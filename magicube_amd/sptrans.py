@@ -218,6 +218,16 @@ def q_csr_softmax(row_indices, row_offsets, values, sqrt_dk: float, scale: float
 # deq_spmm.cpp
 # ---------------------------------------------------------------------------
 
+def _check_groups(slots: int, bits_lhs: int, bits_rhs: int) -> None:
+    """The product reads P and the column indices of a row's last group whole:
+    32 slots with 4-bit V, else 16.  A mask that ends inside a group (and the P
+    that its size asks for) would be read past its end."""
+    group = 32 if bits_rhs == 4 else 16
+    if slots % group:
+        raise ValueError(f"{bits_lhs}-bit P with {bits_rhs}-bit V needs the mask's slots in groups of {group}, "
+                         f"not {slots}")
+
+
 def _bspmm(bits_lhs, bits_rhs, row_indices, row_offsets, column_indices, values, rhs_matrix, vec_length, scale,
            stream):
     _check_v(vec_length)
@@ -232,15 +242,10 @@ def _bspmm(bits_lhs, bits_rhs, row_indices, row_offsets, column_indices, values,
         raise ValueError("values do not split into one P per matrix")
     vals = vals.view(batch, -1)
     nnz = ci.numel()
+    _check_groups(nnz, bits_lhs, bits_rhs)
     need = nnz * vec_length * bits_lhs // 8
     if vals.shape[1] * 4 < need:
         raise ValueError(f"values hold {vals.shape[1] * 4} bytes per matrix; the mask needs {need}")
-    # whole groups of the mask's slots: 32 of 4-bit B's (8 of its index
-    # shuffle), 16 of 16-bit P's
-    group = (32 if bits_lhs == 8 else 8) if bits_rhs == 4 else (16 if bits_lhs == 16 else 1)
-    if nnz % group:
-        raise ValueError(f"{bits_lhs}-bit P with {bits_rhs}-bit V needs the mask's slots in groups of "
-                         f"{32 if bits_rhs == 4 else group}, not {nnz}")
     with _on(stream):
         m = m_vec * vec_length
         out = torch.empty((batch, m, n), dtype=torch.float16, device=rhs.device)

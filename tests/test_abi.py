@@ -191,3 +191,15 @@ def test_spmm_sddmm_mirrors_reject_host_tensors():
         spmm.wmma_spmm(8, 8, 1, 8, 16, 16, None, t, t, t, t, t)
     with pytest.raises(ValueError):
         sddmm.wmma_sddmm(8, 1, 64, 16, None, t, t, t, t, t, 8)
+
+
+@pytest.mark.parametrize("pair,group", [((8, 8), 16), ((16, 8), 16), ((8, 4), 32), ((4, 4), 32)])
+def test_products_refuse_masks_that_end_inside_a_group(pair, group):
+    """The kernel reads whole groups of slots: 40 slots of a (4, 4) product
+    would be 64 column indices and as much P."""
+    from magicube_amd import sptrans
+    for slots in (0, group, 96):
+        sptrans._check_groups(slots, *pair)
+    for slots in (8, 40, group + 1, 96 + group // 2):
+        with pytest.raises(ValueError, match=f"groups of {group}"):
+            sptrans._check_groups(slots, *pair)
