@@ -203,3 +203,61 @@ def test_products_refuse_masks_that_end_inside_a_group(pair, group):
     for slots in (8, 40, group + 1, 96 + group // 2):
         with pytest.raises(ValueError, match=f"groups of {group}"):
             sptrans._check_groups(slots, *pair)
+
+
+def test_layer_entries_validation(mclib):
+    """The attention layer's launches: shapes, widths, strides, null and
+    misaligned pointers (no launch happens)."""
+    P, odd = ctypes.c_void_p(64), ctypes.c_void_p(66)
+
+    def sddmm(bits=8, batch=1, m_vec=4, k=64, n=64, slots=64, ls=0, rs=0, div=1.0, out=P, os=0, V=8, ro=P):
+        return mclib.mc_sddmm_batched_f16(bits, batch, m_vec, k, n, None, ro, P, slots, P, ls, P, rs, div, out, os, V,
+                                          None)
+    assert sddmm(bits=16) == sddmm(k=576) == sddmm(div=0.0) == sddmm(div=2.0 ** 61) == _lib.MC_EUNSUPPORTED
+    assert sddmm(div=float("nan")) == sddmm(div=float("inf")) == _lib.MC_EUNSUPPORTED
+    assert sddmm(bits=12) == _lib.MC_EUNSUPPORTED
+    assert sddmm(V=3) == _lib.MC_EINVAL_V
+    for bad in (dict(slots=-1), dict(k=60), dict(n=0), dict(batch=0), dict(batch=65536), dict(ls=2), dict(os=-1)):
+        assert sddmm(**bad) == _lib.MC_EINVAL_SHAPE, bad
+    for bad in (dict(out=None), dict(out=odd), dict(ro=None), dict(batch=2, os=2)):
+        assert sddmm(**bad) == _lib.MC_EINVAL_ARG, bad
+    assert sddmm(V=2, out=odd) == _lib.MC_EINVAL_ARG
+    assert sddmm(m_vec=0) == _lib.MC_OK
+
+    def spmm(lhs=8, rhs=8, batch=1, m_vec=4, V=8, n=64, k=64, p=P, ps=0, rs=0, out=P, os=0):
+        return mclib.mc_spmm_batched_f16(lhs, rhs, batch, m_vec, V, n, k, None, P, P, p, ps, P, rs, 1.0, out, os, None)
+    for pair in ((12, 8), (16, 16), (12, 4), (16, 4), (4, 8)):
+        assert spmm(*pair) == _lib.MC_EUNSUPPORTED, pair
+    assert spmm(V=3) == _lib.MC_EINVAL_V
+    for bad in (dict(n=6), dict(batch=0), dict(batch=65536), dict(ps=6), dict(rs=-4), dict(os=-1), dict(k=-1)):
+        assert spmm(**bad) == _lib.MC_EINVAL_SHAPE, bad
+    for bad in (dict(out=None), dict(out=odd), dict(p=None), dict(batch=2, os=6)):
+        assert spmm(**bad) == _lib.MC_EINVAL_ARG, bad
+    assert spmm(m_vec=0) == _lib.MC_OK
+
+    assert mclib.mc_attn_quantize(P, 8, 1.0, 16, 0, P, None) == _lib.MC_EUNSUPPORTED
+    assert mclib.mc_attn_quantize(P, 8, 1.0, 8, 4, P, None) == _lib.MC_EINVAL_ARG
+    assert mclib.mc_attn_quantize(P, -1, 1.0, 8, 0, P, None) == _lib.MC_EINVAL_ARG
+    assert mclib.mc_attn_quantize(None, 8, 1.0, 8, 0, P, None) == _lib.MC_EINVAL_ARG
+    assert mclib.mc_attn_quantize(P, 8, 1.0, 8, 0, None, None) == _lib.MC_EINVAL_ARG
+    assert mclib.mc_attn_quantize(None, 0, 1.0, 8, 0, None, None) == _lib.MC_OK
+
+    def gaps(batch=1, rows=4, ro=P, slots=64, group=16, bits=64, out=P, stride=0):
+        return mclib.mc_attn_zero_gaps(batch, rows, ro, slots, group, bits, out, stride, None)
+    for bad in (dict(batch=0), dict(batch=65536), dict(rows=-1), dict(slots=-1), dict(stride=-1)):
+        assert gaps(**bad) == _lib.MC_EINVAL_SHAPE, bad
+    for bad in (dict(group=0), dict(bits=4), dict(bits=12), dict(out=None), dict(ro=None)):
+        assert gaps(**bad) == _lib.MC_EINVAL_ARG, bad
+    assert gaps(slots=0, out=None) == _lib.MC_OK
+
+    def project(L=8, samples=1, heads=4, x=P, w=P, bias=P, qk=8, mats=P, qkv=P):
+        return mclib.mc_attn_in_projection_f16(L, samples, heads, x, w, bias, 36.0, qk, 0, mats, qkv, None)
+    assert project(qk=16) == _lib.MC_EUNSUPPORTED
+    # odd head counts end in half a column tile; 4096 columns, 256 matrices and 2^30 rows at most
+    for bad in (dict(L=-1), dict(samples=0), dict(heads=0), dict(heads=3), dict(heads=22), dict(samples=65),
+                dict(L=1 << 28, samples=4)):
+        assert project(**bad) == _lib.MC_EINVAL_SHAPE, bad
+    for bad in (dict(x=None), dict(w=None), dict(qkv=None), dict(mats=None), dict(x=odd), dict(w=odd), dict(bias=odd),
+                dict(qkv=odd)):
+        assert project(**bad) == _lib.MC_EINVAL_ARG, bad
+    assert project(L=0, x=None) == _lib.MC_OK
