@@ -122,23 +122,27 @@ def _bsddmm(bits, row_indices, row_offsets, column_indices, lhs_matrix, rhs_matr
         raise ValueError("lhs_matrix and rhs_matrix must share k")
     if m != m_vec * vec_length:
         raise ValueError(f"lhs_matrix has {m} rows; the mask covers {m_vec} vector rows of {vec_length}")
-    nnz = ci.numel()
+    # rows are written up to a multiple of 8 slots: of a mask that ends inside
+    # such a group, past its last slot
+    nnz, slots = ci.numel(), -(-ci.numel() // 8) * 8
     with _on(stream):
-        out = torch.empty((batch, nnz * vec_length) if batched else (nnz * vec_length,), dtype=torch.float16,
-                          device=lhs.device)
+        full = torch.empty((batch, slots * vec_length), dtype=torch.float16, device=lhs.device)
+        out = full if slots == nnz else full[:, :nnz * vec_length]
         lib, st = _lib.lib(), _stream_handle(stream)
         # K in one pass and a divisor the kernel's quotient covers: it stores fp16 itself
         if k <= 512 and m_vec and 2.0 ** -60 <= abs(scale) <= 2.0 ** 60:
-            _lib.check(lib.mc_sddmm_batched_f16(bits, batch, m_vec, k, n, _ptr(ri), _ptr(ro), _ptr(ci), nnz,
+            _lib.check(lib.mc_sddmm_batched_f16(bits, batch, m_vec, k, n, _ptr(ri), _ptr(ro), _ptr(ci), slots,
                                                 _ptr(lhs), m * k_int32 * 4, _ptr(rhs), n * k_int32 * 4, float(scale),
-                                                _ptr(out), nnz * vec_length, vec_length, st), f"bsddmm_{bits}b")
-            return out
-        acc = torch.zeros((batch, nnz * vec_length), dtype=torch.int32, device=lhs.device)
-        _lib.check(lib.mc_sddmm_batched(bits, _lib.MC_SIGNED, 1, batch, m_vec, k, n, _ptr(ri), _ptr(ro), _ptr(ci),
-                                        _ptr(lhs), m * k_int32 * 4, _ptr(rhs), n * k_int32 * 4, _ptr(acc),
-                                        nnz * vec_length, vec_length, st), f"bsddmm_{bits}b")
-        _lib.check(lib.mc_attn_dequant_f16(_ptr(acc), acc.numel(), float(scale), _ptr(out), st), "bsddmm dequant")
-    return out
+                                                _ptr(full), slots * vec_length, vec_length, st), f"bsddmm_{bits}b")
+        else:
+            acc = torch.zeros((batch, slots * vec_length), dtype=torch.int32, device=lhs.device)
+            _lib.check(lib.mc_sddmm_batched(bits, _lib.MC_SIGNED, 1, batch, m_vec, k, n, _ptr(ri), _ptr(ro), _ptr(ci),
+                                            _ptr(lhs), m * k_int32 * 4, _ptr(rhs), n * k_int32 * 4, _ptr(acc),
+                                            slots * vec_length, vec_length, st), f"bsddmm_{bits}b")
+            _lib.check(lib.mc_attn_dequant_f16(_ptr(acc), acc.numel(), float(scale), _ptr(full), st), "bsddmm dequant")
+        if not batched:
+            return out.view(-1)
+        return out if slots == nnz else out.contiguous()
 
 
 def bsddmm_8b(row_indices, row_offsets, column_indices, lhs_matrix, rhs_matrix, vec_length: int, bits: int,
@@ -192,20 +196,25 @@ def q_bcsr_softmax(row_indices, row_offsets, values, sqrt_dk: float, scale: floa
     if (stride * bits) % 32:
         raise ValueError(f"{stride} values per matrix do not pack into int32 words of {bits}-bit P")
     attn_stride = stride * bits // 32
+    # rows are written in whole groups of slots: of a mask that ends inside
+    # one, past its last slot
+    group = 32 if bits == 4 else 16
+    slots = -(-stride // (group * vec_length)) * group
+    full_stride = slots * vec_length * bits // 32
     with _on(stream):
         lib, st = _lib.lib(), _stream_handle(stream)
-        rows, slots = ri.numel(), stride // vec_length
-        if 2 * rows == ro.numel() and stride % vec_length == 0:
+        rows = ri.numel()
+        if 2 * rows == ro.numel():
             # every row is written: only the slots between rows need zeros
-            attn = torch.empty((batch_size, attn_stride), dtype=torch.int32, device=vals.device)
-            _lib.check(lib.mc_attn_zero_gaps(batch_size, rows, _ptr(ro), slots, 32 if bits == 4 else 16,
-                                             vec_length * bits, _ptr(attn), attn_stride * 4, st), "q_bcsr_softmax")
+            attn = torch.empty((batch_size, full_stride), dtype=torch.int32, device=vals.device)
+            _lib.check(lib.mc_attn_zero_gaps(batch_size, rows, _ptr(ro), slots, group, vec_length * bits, _ptr(attn),
+                                             full_stride * 4, st), "q_bcsr_softmax")
         else:
-            attn = torch.zeros((batch_size, attn_stride), dtype=torch.int32, device=vals.device)
+            attn = torch.zeros((batch_size, full_stride), dtype=torch.int32, device=vals.device)
         _lib.check(lib.mc_attn_softmax_f16(batch_size, rows, vec_length, _ptr(ri), _ptr(ro), _ptr(vals), stride,
-                                           float(sqrt_dk), float(scale), bits, _ptr(attn), attn_stride * 4, st),
+                                           float(sqrt_dk), float(scale), bits, _ptr(attn), full_stride * 4, st),
                    "q_bcsr_softmax")
-    return attn
+        return attn if full_stride == attn_stride else attn[:, :attn_stride].contiguous()
 
 
 def q_csr_softmax(row_indices, row_offsets, values, sqrt_dk: float, scale: float, vec_length: int, bits: int,

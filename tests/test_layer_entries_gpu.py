@@ -275,3 +275,58 @@ def test_in_projection_entry(heads, samples, L, qk_bits, range4, bias):
     # an fp16 y differs from the exact one's rounding at about 1 in 500 for the
     # longest sums, a truncation then at less than 1 in 10
     assert wrong <= total // 1000
+
+
+@pytest.fixture
+def guarded(monkeypatch):
+    """Every tensor that torch.empty and torch.zeros allocate is followed by a guard."""
+    made = []
+
+    def guarded_fill(fill):
+        def make(shape, dtype, device):
+            n = int(np.prod(shape))
+            size = n * dtype.itemsize
+            buf = torch.full((size + 8 * GUARD,), FILL, dtype=torch.uint8, device=device)
+            buf[:size] = fill
+            made.append((buf, size))
+            return buf[:size].view(dtype).view(shape)
+        return make
+
+    def check():
+        torch.cuda.synchronize()
+        assert made and all((buf[size:] == FILL).all() for buf, size in made), "written past the end"
+
+    monkeypatch.setattr(torch, "empty", guarded_fill(FILL))
+    monkeypatch.setattr(torch, "zeros", guarded_fill(0))
+    yield check
+    monkeypatch.undo()
+
+
+@pytest.mark.parametrize("V", [8, 4, 2])
+@pytest.mark.parametrize("last", [1, 9, 20, 36, 41])
+def test_masks_that_end_inside_a_group(V, last, guarded):
+    """The last row's slots are the mask's last (no padding up to a multiple of
+    8, 16 or 32): the ops answer for these slots what they answer for the same
+    mask with its padding, and store nothing past their outputs."""
+    counts = COUNTS + (last,)
+    order, pairs, cols = ragged_mask(32, seed=V + last, counts=counts)
+    cut = int(pairs[-1])
+    assert cut % 8 and cut + 31 >= cols.size
+    short = cols[:cut]
+    rng = np.random.default_rng(V)
+    for k in (64, 576):                        # fp16 stored by the kernel; int32 and a second pass
+        lhs = rng.integers(-8, 8, size=(2, len(counts) * V, k))
+        rhs = rng.integers(-8, 8, size=(2, KEYS, k))
+        ri, ro, a, b = dev(order), dev(pairs), packed(lhs, 8), packed(rhs, 8)
+        whole = sptrans.bsddmm_8b(ri, ro, dev(cols), a, b, V, 8, 324.0)
+        got = sptrans.bsddmm_8b(ri, ro, dev(short), a, b, V, 8, 324.0)
+        one = sptrans.sddmm_8b(ri, ro, dev(short), a[0], b[0], V, 8, 324.0)
+        assert got.is_contiguous() and torch.equal(got, whole[:, :cut * V]) and torch.equal(one, got[0])
+    logits = whole
+    for bits in (16, 8, 4):
+        if cut * V * bits % 32:
+            continue                           # refused: no whole number of words
+        exp = sptrans.q_bcsr_softmax(ri, ro, logits, 0.125, 7.0, V, 2, bits)
+        got = sptrans.q_bcsr_softmax(ri, ro, logits[:, :cut * V], 0.125, 7.0, V, 2, bits)
+        assert got.is_contiguous() and torch.equal(got, exp[:, :cut * V * bits // 32])
+    guarded()
