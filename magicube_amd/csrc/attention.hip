@@ -37,6 +37,16 @@ typedef __attribute__((address_space(1))) const v4i global_v4i;
 typedef __attribute__((address_space(1))) v2i global_v2i;
 typedef __attribute__((address_space(1))) u32 global_u32;
 
+__device__ __forceinline__ void unpack_half8(const v4i &w, float (&x)[8]) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int we = w[e];
+        const __half2 h2 = *reinterpret_cast<const __half2 *>(&we);
+        x[2 * e] = __low2float(h2);
+        x[2 * e + 1] = __high2float(h2);
+    }
+}
+
 // 8 values -> 8 int8 or packed int4 at group gi of the job's output
 template <int BITS>
 __device__ __forceinline__ void quantize_group(const float (&x)[8], const QuantJob &jb, int rounding, float lo,
@@ -95,26 +105,40 @@ template <int BITS> __device__ __forceinline__ void quantize_job(const QuantJob 
 #pragma unroll
             for (int k = 0; k < G; ++k) {
                 float x[8];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int we = w[k][e];
-                    const __half2 h2 = *reinterpret_cast<const __half2 *>(&we);
-                    x[2 * e] = __low2float(h2);
-                    x[2 * e + 1] = __high2float(h2);
-                }
+                unpack_half8(w[k], x);
                 if (g0 + 256 * k < done) quantize_group<BITS>(x, jb, rounding, lo, hi, g0 + 256 * k);
             }
         }
     }
-    // the rest value by value: the last part of a group, unaligned or
-    // irregular rows (8 values never straddle a source row: row_len % 8 == 0)
-    for (long long gi = done + (long long)blockIdx.x * 256 + threadIdx.x; gi < groups; gi += (long long)gridDim.x * 256) {
-        const long long base = gi * 8;
-        const __half *src = jb.row_len ? jb.x + (base / jb.row_len) * jb.row_stride + base % jb.row_len : jb.x + base;
-        float x[8];
+    // the rest: the last part of a group, and jobs of other row lengths or
+    // alignments (8 values never straddle a source row: row_len % 8 == 0), 16
+    // bytes at a time where a group's source allows it: 32768 rows of 96 or 80
+    // values take 4.5 us, value by value 5.8 and 5.6
+    for (long long blk = blockIdx.x; done + blk * 256 * G < groups; blk += gridDim.x) {
+        const long long g0 = done + blk * 256 * G + threadIdx.x;
+        v4i w[G];
+        const __half *src[G];
+        bool vec[G];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = base + e < jb.count ? __half2float(src[e]) : 0.f;
-        quantize_group<BITS>(x, jb, rounding, lo, hi, gi);
+        for (int k = 0; k < G; ++k) {
+            const long long base = (g0 + 256 * k) * 8;
+            src[k] = jb.row_len ? jb.x + (base / jb.row_len) * jb.row_stride + base % jb.row_len : jb.x + base;
+            vec[k] = base + 8 <= jb.count && (reinterpret_cast<uintptr_t>(src[k]) & 15u) == 0;
+            if (vec[k]) w[k] = __builtin_nontemporal_load((global_v4i *)src[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < G; ++k) {
+            const long long gi = g0 + 256 * k;
+            if (gi >= groups) continue;
+            float x[8];
+            if (vec[k]) {
+                unpack_half8(w[k], x);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = gi * 8 + e < jb.count ? __half2float(src[k][e]) : 0.f;
+            }
+            quantize_group<BITS>(x, jb, rounding, lo, hi, gi);
+        }
     }
 }
 

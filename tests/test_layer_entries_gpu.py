@@ -115,6 +115,25 @@ def test_quantize_one(bits, count):
     assert np.array_equal(lanes, oatt.quantize_ref(x.cpu().numpy(), 30.0, bits, 0).ravel())
 
 
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("row_len,stride,offset", [(96, 288, 0), (80, 84, 0), (48, 200, 4), (8, 24, 0), (40, 40, 1),
+                                                   (64, 196, 0), (0, 0, 4), (0, 0, 0)])
+def test_quantize_row_lengths(bits, row_len, stride, offset):
+    """Jobs whose rows are no power of two, or start off 16 bytes."""
+    rows = 701
+    count = rows * row_len if row_len else 701 * 24 + (0 if bits == 4 else 3)
+    x = torch.randn(rows * max(stride, 32) + offset, device="cuda").half()
+    src = x[offset:].cpu().numpy()
+    src = np.stack([src[i * stride:i * stride + row_len] for i in range(rows)]).ravel() if row_len else src[:count]
+    out = Owned(count * bits // 8)
+    job = attention._QuantJobC(x.data_ptr() + 2 * offset, count, 30.0, out.ptr, row_len, stride)
+    jobs = torch.frombuffer(bytearray(bytes(job)), dtype=torch.uint8).cuda()
+    _lib.check(_lib.lib().mc_attn_quantize_batched(jobs.data_ptr(), 1, bits, attention.ROUND_TRUNC, count, stream()),
+               "quantize_batched")
+    lanes = formats.unpack_lanes(out.bytes(), bits, count, signed=True)
+    assert np.array_equal(lanes, oatt.quantize_ref(src, 30.0, bits, 0))
+
+
 @pytest.fixture
 def poisoned(monkeypatch):
     """torch.empty hands out memory full of FILL."""
