@@ -15,21 +15,28 @@ int mfma_rows(int lhs_bits, int rhs_bits, bool sgn, int V) {
 }
 
 int default_config(int rhs_bits, int n, long long m_vec, int rows) {
-    // Four dwords of 8- or 16-bit B per lane where the launch fills the GPU
-    // with such tiles (2048 waves of 16 * 4 dwords) and a vector row is one MFMA row tile
-    // (two need 128 accumulators and leave two waves per SIMD).  The gathers
-    // are bound by L1's address path: a 4-byte load of a wave takes it 8
-    // cycles, a 16-byte one 16.  Measured on MI355X, us, one dword and four
-    // waves per row (config 17) against this: L8-R8, V = 8, 8192 x 8192, N =
-    // 4096, 90 % sparse 261 / 160; 4096 x 4096, N = 4096, 70, 90, 98 % 147 /
-    // 112, 59 / 45, 20.3 / 19.4; N = 2048, 90 % 33.5 / 25.6; N = 1024, 70, 90,
-    // 98 % 43 / 32, 16.8 / 14.6, 7.9 / 8.1; N = 512 (1024 waves) 24.0 / 25.2,
-    // 10.1 / 11.7, 6.4 / 6.9.  L16-R8, V = 4, N = 4096, 80 and 95 % 103 / 74,
-    // 32 / 30; L16-R16, V = 4 252 / 154, 77 / 61.  Two row tiles: L16-R8, V =
-    // 8 114 / 135, 42 / 62 (config 25: 99, 55).
+    // Four dwords of 8- or 16-bit B per lane where the launch holds 2048 waves
+    // of 16 * 4 dwords, two per workgroup (an odd tile's second wave included),
+    // and a vector row is one MFMA row tile (two need 128 accumulators and
+    // leave two waves per SIMD).  The gathers are bound by L1's address path:
+    // a 4-byte load of a wave takes it 8 cycles, a 16-byte one 16.  Measured on
+    // MI355X, us, one dword and four waves per row (config 17) against this:
+    // L8-R8, V = 8, 8192 x 8192, N = 4096, 90 % sparse 261 / 160; 4096 x 4096,
+    // N = 4096, 70 and 90 % 147 / 112, 59 / 45; N = 2048, 90 % 33.5 / 25.6; N =
+    // 1024, 70 and 90 % 43 / 32, 16.8 / 14.6; N = 512 (1024 waves) 24.0 / 25.2,
+    // 10.1 / 11.7.  L16-R8, V = 4, N = 4096, 80 % 103 / 74; L16-R16, V = 4 252 /
+    // 154.  Two row tiles: L16-R8, V = 8 114 / 135, 42 / 62 (config 25: 99, 55).
+    // Not for a row of three tiles: the fourth wave has no columns and the
+    // third few just past the second, where config 17 fills its waves better
+    // (1024 vector rows, K = 4096, 90 %: N = 516 26.0 / 28.5, 580 28.7 / 28.4,
+    // 640 22.5 / 25.3, 768 24.0 / 25.9; 512 rows 14.0 / 16.5, 16.1 / 16.9, 13.0
+    // / 14.1, 14.3 / 14.4).  Two tiles and four or five are faster from their
+    // first column on (1024 rows: 260 20.0 / 13.7, 320 16.3 / 13.4, 772 37.4 /
+    // 29.0, 1028 50.8 / 38.6; 512 rows: 772 19.9 / 17.3, 1028 27.9 / 21.7).
     if (rhs_bits != 4 && rows <= 16 && n % 4 == 0 && n >= 4 * (32 / rhs_bits)) {
         const int wide = 64 * (32 / rhs_bits);
-        if (m_vec * 2 * ((n + 2 * wide - 1) / (2 * wide)) >= 2048 && n > wide) return 24;
+        const int wide_tiles = (n + wide - 1) / wide;
+        if (m_vec * 2 * ((wide_tiles + 1) / 2) >= 2048 && wide_tiles > 1 && wide_tiles != 3) return 24;
     }
     // One dword of B per lane and one k-block of gathers in flight per wave:
     // latency is hidden by more resident waves rather than deeper per-wave
@@ -209,6 +216,13 @@ mc_status mc_spmm_get_tile_config(int index, mc_tile_config *out) {
     if (index < 0 || index >= mc::kNumSpmmConfigs || !out) return MC_EINVAL_ARG;
     *out = mc::kSpmmConfigs[index];
     return MC_OK;
+}
+
+int mc_spmm_default_config(int lhs_bits, int rhs_bits, mc_signedness sign, int m_vec, int vec_length, int n) {
+    if (!mc::pair_supported(lhs_bits, rhs_bits) || !mc::valid_v(vec_length) || m_vec < 0 || n <= 0 ||
+        n % (32 / rhs_bits) != 0)
+        return -1;
+    return mc::default_config(rhs_bits, n, m_vec, mc::mfma_rows(lhs_bits, rhs_bits, sign == MC_SIGNED, vec_length));
 }
 
 mc_status mc_spmm_run(int lhs_bits, int rhs_bits, mc_signedness sign, int config, int m_vec, int vec_length, int n,
