@@ -14,7 +14,9 @@ int mfma_rows(int lhs_bits, int rhs_bits, bool sgn, int V) {
     return (lhs_bits / 4 - (sgn ? 1 : 0)) * V;
 }
 
-int default_config(int rhs_bits, int n, long long m_vec, int rows) {
+// row_slots: nonzero vectors per vector row on average, 0 where the caller does
+// not know.
+int default_config(int rhs_bits, int n, long long m_vec, int rows, int row_slots) {
     // Four dwords of 8- or 16-bit B per lane where the launch holds 2048 waves
     // of 16 * 4 dwords, two per workgroup (an odd tile's second wave included),
     // and a vector row is one MFMA row tile (two need 128 accumulators and
@@ -33,10 +35,20 @@ int default_config(int rhs_bits, int n, long long m_vec, int rows) {
     // / 14.1, 14.3 / 14.4).  Two tiles and four or five are faster from their
     // first column on (1024 rows: 260 20.0 / 13.7, 320 16.3 / 13.4, 772 37.4 /
     // 29.0, 1028 50.8 / 38.6; 512 rows: 772 19.9 / 17.3, 1028 27.9 / 21.7).
+    // Nor for short rows of 8-bit B, whose gathers cost less than the fewer
+    // waves and the store through LDS: the launch then has to be larger.  17 /
+    // this at 32, 96, 192, 256 and 400 slots per row: 1024 x 4096, N = 1024,
+    // L8-R8, V = 8 9.4 / 10.5, 11.9 / 13.2, 16.8 / 17.4, 21.0 / 21.0, 30.6 /
+    // 26.9; L16-R8, V = 4 12.4 / 13.1, 13.6 / 15.5, 17.5 / 19.2, 20.8 / 22.0,
+    // 30.1 / 27.1; N = 2048 15.2 / 17.4, 20.9 / 21.1, 33.1 / 31.5, 40.8 / 36.3,
+    // 60.1 / 47.0; N = 4096 (16384 waves) 30.4 / 31.8, 42.2 / 38.5, 63.9 / 53.7.
+    // 16-bit B is faster at every length (14.6 / 13.0, 16.1 / 16.0, 32.6 / 29.4).
     if (rhs_bits != 4 && rows <= 16 && n % 4 == 0 && n >= 4 * (32 / rhs_bits)) {
         const int wide = 64 * (32 / rhs_bits);
         const int wide_tiles = (n + wide - 1) / wide;
-        if (m_vec * 2 * ((wide_tiles + 1) / 2) >= 2048 && wide_tiles > 1 && wide_tiles != 3) return 24;
+        const long long waves = m_vec * 2 * ((wide_tiles + 1) / 2);
+        const int least = rhs_bits == 16 || waves >= 16384 ? 0 : waves >= 8192 ? 192 : 320;
+        if (waves >= 2048 && wide_tiles > 1 && wide_tiles != 3 && (row_slots == 0 || row_slots >= least)) return 24;
     }
     // One dword of B per lane and one k-block of gathers in flight per wave:
     // latency is hidden by more resident waves rather than deeper per-wave
@@ -88,7 +100,8 @@ mc_status spmm_entry(int lhs_bits, int rhs_bits, mc_signedness sign, int config,
                      int k, const int *row_indices, const int *row_offsets, const int *column_indices,
                      const int *values, const int *rhs_matrix, int *output_matrix, hipStream_t stream,
                      int batch = 1, long long values_stride = 0, long long rhs_stride = 0,
-                     long long out_stride = 0, __half *out16 = nullptr, float divisor = 1.f) {
+                     long long out_stride = 0, __half *out16 = nullptr, float divisor = 1.f,
+                     int row_slots = 0) {
     if (!pair_supported(lhs_bits, rhs_bits)) return MC_EUNSUPPORTED;
     if (batch < 1 || batch > 65535 || values_stride < 0 || rhs_stride < 0 || out_stride < 0) return MC_EINVAL_SHAPE;
     if ((values_stride | rhs_stride) & 3) return MC_EINVAL_SHAPE;   // every matrix starts dword aligned
@@ -105,7 +118,7 @@ mc_status spmm_entry(int lhs_bits, int rhs_bits, mc_signedness sign, int config,
     if (config < -1 || config >= kNumSpmmConfigs) return MC_EINVAL_ARG;
     // a batched launch fills the GPU with (row, tile) x batch workgroups
     const int rows = out16 ? 32 : mfma_rows(lhs_bits, rhs_bits, sign == MC_SIGNED, vec_length);
-    int cfg = config >= 0 ? config : default_config(rhs_bits, n, (long long)m_vec * batch, rows);
+    int cfg = config >= 0 ? config : default_config(rhs_bits, n, (long long)m_vec * batch, rows, row_slots);
     if (!config_supported(cfg, rhs_bits)) return MC_EUNSUPPORTED;
     if (batch > 1 && kSpmmConfigs[cfg].kind == 1) return MC_EUNSUPPORTED;   // B-stationary: one matrix
     if (kSpmmConfigs[cfg].kind == 1 && !stationary_fits(cfg, n, k)) {
@@ -218,11 +231,22 @@ mc_status mc_spmm_get_tile_config(int index, mc_tile_config *out) {
     return MC_OK;
 }
 
-int mc_spmm_default_config(int lhs_bits, int rhs_bits, mc_signedness sign, int m_vec, int vec_length, int n) {
+int mc_spmm_default_config(int lhs_bits, int rhs_bits, mc_signedness sign, int m_vec, int vec_length, int n,
+                           int row_slots) {
     if (!mc::pair_supported(lhs_bits, rhs_bits) || !mc::valid_v(vec_length) || m_vec < 0 || n <= 0 ||
-        n % (32 / rhs_bits) != 0)
+        n % (32 / rhs_bits) != 0 || row_slots < 0)
         return -1;
-    return mc::default_config(rhs_bits, n, m_vec, mc::mfma_rows(lhs_bits, rhs_bits, sign == MC_SIGNED, vec_length));
+    return mc::default_config(rhs_bits, n, m_vec, mc::mfma_rows(lhs_bits, rhs_bits, sign == MC_SIGNED, vec_length),
+                              row_slots);
+}
+
+mc_status mc_spmm_run_rows(int lhs_bits, int rhs_bits, mc_signedness sign, int row_slots, int m_vec, int vec_length,
+                           int n, int k, const int *row_indices, const int *row_offsets, const int *column_indices,
+                           const int *values, const int *rhs_matrix, int *output_matrix, hipStream_t stream) {
+    if (row_slots < 0) return MC_EINVAL_ARG;
+    return mc::spmm_entry(lhs_bits, rhs_bits, sign, -1, m_vec, vec_length, n, k, row_indices, row_offsets,
+                          column_indices, values, rhs_matrix, output_matrix, stream, 1, 0, 0, 0, nullptr, 1.f,
+                          row_slots);
 }
 
 mc_status mc_spmm_run(int lhs_bits, int rhs_bits, mc_signedness sign, int config, int m_vec, int vec_length, int n,

@@ -83,6 +83,15 @@ def _check_device(tensors, what: str) -> None:
     raise ValueError(f"{what}: operands are on several devices {sorted(map(str, devs))}")
 
 
+def _row_slots(rhs_bits: int, m_vec: int, n: int, column_indices) -> int:
+    """Slots per vector row on average where the default tile depends on it
+    (short rows of 8-bit B over more columns than one wide tile), else 0."""
+    if rhs_bits != 8 or n <= 256 or not isinstance(column_indices, torch.Tensor):
+        return 0
+    slots = column_indices.numel() // max(m_vec, 1)
+    return max(slots, 1) if slots < 320 else 0
+
+
 def wmma_spmm(lhs_bits: int, rhs_bits: int, m_vec: int, vec_length: int, n: int, k: int, row_indices,
               row_offsets, column_indices, values, rhs_matrix, output_matrix, sign: int = SIGNED,
               config: int | None = None, stream=None) -> None:
@@ -94,8 +103,12 @@ def wmma_spmm(lhs_bits: int, rhs_bits: int, m_vec: int, vec_length: int, n: int,
     args = (m_vec, vec_length, n, k, _dptr(row_indices), _dptr(row_offsets), _dptr(column_indices),
             _dptr(values), _dptr(rhs_matrix), _dptr(output_matrix))
     if config is None:
-        fn = getattr(lib, _PAIR_FN[(lhs_bits, rhs_bits)])
-        st = fn(*args, sign, _stream(stream))
+        slots = _row_slots(rhs_bits, m_vec, n, column_indices) if n > 256 else 0
+        if slots:
+            st = lib.mc_spmm_run_rows(lhs_bits, rhs_bits, sign, slots, *args, _stream(stream))
+        else:
+            fn = getattr(lib, _PAIR_FN[(lhs_bits, rhs_bits)])
+            st = fn(*args, sign, _stream(stream))
     else:
         st = lib.mc_spmm_run(lhs_bits, rhs_bits, sign, config, *args, _stream(stream))
     _lib.check(st, f"spmm L{lhs_bits}-R{rhs_bits}")

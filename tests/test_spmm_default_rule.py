@@ -10,12 +10,14 @@ def mfma_rows(lhs, signed, V):
     return planes * V
 
 
-def restated(lhs, rhs, signed, m_vec, V, n):
+def restated(lhs, rhs, signed, m_vec, V, n, slots):
     wide = 256 if rhs == 8 else 128
     tiles = -(-n // wide)
     if rhs != 4 and n % 4 == 0 and mfma_rows(lhs, signed, V) <= 16:
         # the rows' waves in workgroups of two; three tiles leave one of four without columns
-        if tiles in (2,) + tuple(range(4, 100)) and m_vec * (tiles + tiles % 2) >= 2048:
+        waves = m_vec * (tiles + tiles % 2)
+        short = rhs == 8 and 0 < slots < 320 and waves < 16384 and not (waves >= 8192 and slots >= 192)
+        if tiles in (2,) + tuple(range(4, 100)) and waves >= 2048 and not short:
             return 24
     cols = 16 * (32 // rhs)
     narrow = -(-n // cols)
@@ -39,21 +41,40 @@ def test_default_tile(mclib, pair):
         for m_vec in (1, 63, 255, 256, 257, 341, 342, 511, 512, 513, 1023, 1024, 2048, 4096):
             for V in (2, 4, 8):
                 for signed in (True, False):
-                    got = mclib.mc_spmm_default_config(lhs, rhs, 0 if signed else 1, m_vec, V, n)
-                    assert got == restated(lhs, rhs, signed, m_vec, V, n), (pair, n, m_vec, V, signed)
-                    seen.add(got)
+                    for slots in (0, 1, 191, 192, 319, 320):
+                        got = mclib.mc_spmm_default_config(lhs, rhs, 0 if signed else 1, m_vec, V, n, slots)
+                        assert got == restated(lhs, rhs, signed, m_vec, V, n, slots), (pair, n, m_vec, V, signed, slots)
+                        seen.add(got)
     assert seen == ({13, 15, 16, 17, 20, 22} | ({24} if rhs != 4 else set()))
 
 
 def test_three_wide_tiles_are_not_four(mclib):
     """516 to 768 columns are three tiles of 256: a quarter of the waves would have no columns."""
     for n in (516, 580, 640, 768):
-        assert mclib.mc_spmm_default_config(8, 8, 0, 512, 8, n) == 17
-        assert mclib.mc_spmm_default_config(8, 8, 0, 1024, 8, n) == 17
+        assert mclib.mc_spmm_default_config(8, 8, 0, 512, 8, n, 0) == 17
+        assert mclib.mc_spmm_default_config(8, 8, 0, 1024, 8, n, 0) == 17
     for n in (512, 772, 1028):
-        assert mclib.mc_spmm_default_config(8, 8, 0, 1024, 8, n) == 24
+        assert mclib.mc_spmm_default_config(8, 8, 0, 1024, 8, n, 0) == 24
+
+
+def test_short_rows_of_a_resident_operand(mclib):
+    """What the Python products pass on: the slots of the index array, and
+    nothing where the tile does not depend on them."""
+    import torch
+    from magicube_amd import _lib, spmm
+    cols = torch.zeros(1024 * 82, dtype=torch.int32)
+    assert spmm._row_slots(8, 1024, 1024, cols) == 82
+    assert mclib.mc_spmm_default_config(8, 8, 0, 1024, 8, 1024, 82) == 17
+    assert spmm._row_slots(8, 1024, 1024, cols[:16]) == 1
+    for args in ((16, 1024, 1024, cols), (4, 1024, 1024, cols), (8, 1024, 256, cols), (8, 256, 1024, cols),
+                 (8, 1024, 1024, 1 << 20), (8, 0, 1024, cols)):
+        assert spmm._row_slots(*args) == 0
+    p = 64
+    assert mclib.mc_spmm_run_rows(8, 8, 0, -1, 4, 8, 64, 64, None, p, p, p, p, p, None) == _lib.MC_EINVAL_ARG
+    assert mclib.mc_spmm_run_rows(8, 8, 0, 82, 0, 8, 64, 64, None, p, p, p, p, p, None) == _lib.MC_OK
 
 
 def test_refused_arguments_have_no_tile(mclib):
-    for args in ((12, 16, 0, 4, 8, 64), (8, 8, 0, 4, 3, 64), (8, 8, 0, -1, 8, 64), (8, 8, 0, 4, 8, 0), (8, 8, 0, 4, 8, 6)):
+    for args in ((12, 16, 0, 4, 8, 64, 0), (8, 8, 0, 4, 3, 64, 0), (8, 8, 0, -1, 8, 64, 0), (8, 8, 0, 4, 8, 0, 0),
+                 (8, 8, 0, 4, 8, 6, 0), (8, 8, 0, 4, 8, 64, -1)):
         assert mclib.mc_spmm_default_config(*args) == -1
