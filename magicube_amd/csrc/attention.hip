@@ -529,10 +529,11 @@ __device__ __forceinline__ int const_load(const int *p) {
 // V + 8 (0..15), so the MFMA forms P (V + 8) and 8 * (row sum of P) comes off
 // the accumulators at the end (exact mod 2^32).
 //
-// Bound by the address and data path of L1 (TA / TD busy three quarters of the
-// kernel) with VALU issue close behind, not by L2: sending every gather to one
-// 4 KB window takes the same time, dropping the arithmetic or the gathers does
-// not.  So each logit is scaled, exponentiated and summed once: pass 1 needs
+// Bound by the address and data path of L1 with VALU issue close behind, not by
+// L2: sending every gather to one 4 KB window takes the same time, dropping the
+// arithmetic or the gathers does not.  Counters: TD busy 89 % of the time (36 %
+// of that waiting for L2), TA 78, VALU 69, LDS 36 over 128 matrices of L up to
+// 4096, row-scaled P; 81, 68, 67 and 42 % over 32 of L = 4096, reference P.  So each logit is scaled, exponentiated and summed once: pass 1 needs
 // the max alone, its logits go to pass 2 through LDS (the first SST chunks)
 // and registers (two more); lanes keep their own sums, reduced once per row;
 // the real rows sit in all four lane groups of the MFMA tile; four P bytes are

@@ -24,12 +24,11 @@
 // sum against its own running max, rescaled when that grows, and brings it to
 // the row max before the tree.  Both kernels evaluate these statistics on the
 // same register layout (MFMA C layout: lane (c, g) holds rows 4g+i of
-// slot 16t + c) with the same instructions.  The fused kernel first moves
-// the V real rows out of the MFMA tile's padding lanes (rows are dealt to
-// the four 16-lane groups instead of four rows per group), so it keeps fewer
-// rows per lane; each row is still held by the 16 lanes c of one group with
-// slots 16t + c, and its statistics take the same operations in the same
-// order.
+// slot 16t + c) with the same instructions.  The fused kernel deals the V
+// real rows to the four 16-lane groups as it loads Q (tile rows 4q + j), so
+// it keeps fewer rows per lane and moves none; each row is still held by the
+// 16 lanes c of one group with slots 16t + c, and its statistics take the
+// same operations in the same order.
 #pragma once
 
 #include <hip/hip_fp16.h>

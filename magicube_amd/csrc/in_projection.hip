@@ -50,14 +50,16 @@ __device__ __forceinline__ int as_int(const __half2 &x) { return *reinterpret_ca
 // while a stage is multiplied or a tile stored.  An XCD takes whole row
 // blocks, so that x crosses HBM once and the column blocks read it from L2.
 //
-// 32768 rows of 256 to 768 take 30 us (kernel trace), where torch's product and
-// the quantize launch took 27 and 12; a batch-8 attention
-// module of L = 4096, E = 256 went from 126.6 to 107.0 us.  MFMA, LDS and L1
-// are each busy about a quarter of the time (rows of 512 to 1536), without
-// bank conflicts.  Not faster: two stages' loads kept in flight over the
-// barrier, the next stage written to LDS under the products, three workgroups
-// per CU with 32-deep stages, 256-row tiles; one and a half workgroups per CU
-// cost 6 us, one tile per workgroup 5.
+// 32768 rows of 256 to 768 take 30 us in a kernel trace and 27 in a row, where
+// torch's product takes 27 and a quantize launch of K and V 10 to 12 (one after
+// the other 40); a batch-8 attention module of L = 4096, E = 256 went from 126.6
+// to 107.0 us.  There TD is busy 44 % of the time (57 % of it waiting), TA 31,
+// VALU 24, LDS 16 without bank conflicts, MFMA 15: bound by the latency of its
+// stages.  At that size one and a half workgroups per CU take 33-35 us and one
+// tile per workgroup 28-30 against 27-28.  By passes of the module, two stages'
+// loads kept in flight over the barrier, the next stage written to LDS under
+// the products, three workgroups per CU with 32-deep stages and 256-row tiles
+// were 0-2 % slower.
 template <int KB>
 __global__ __launch_bounds__(256, 2) void in_projection_kernel(ProjectionArgs a, int mb, int nb) {
     __shared__ v4i xs[2][kTileM * 8], ws[2][kTileN * 8];

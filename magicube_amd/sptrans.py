@@ -31,6 +31,9 @@ reference feeds its signed quantized Q/K/V to unsigned tensor-core MMAs
 which changes its results wherever a lane is negative; these ops compute the
 signed products the layer means.
 
+``row_indices`` is a permutation of the mask's vector rows: every row is written
+once, and only the slots between rows are zeroed beside them.
+
 Each product is one launch (``mc_spmm_batched_f16``): the kernel reads P as
 the softmax op writes it and the mask's indices in their natural order, and
 divides and rounds to fp16 as it stores.
