@@ -125,17 +125,18 @@ mc_status mc_spmm_get_tile_config(int index, mc_tile_config *out);
 /* Config index that a product with the default tile runs: four dwords of 8- or
  * 16-bit B per lane for wide products; else one, up to four (eight) waves per
  * row as n allows, and the row's k-blocks split over two waves when the launch
- * would hold fewer than 2048 waves.  row_slots: nonzero vectors per vector row
- * on average (0: not known).  -1 for arguments that a product refuses. */
-int mc_spmm_default_config(int lhs_bits, int rhs_bits, mc_signedness sign, int m_vec, int vec_length, int n,
+ * would hold fewer than 2048 waves.  row_slots: slots per vector row on
+ * average (0: not known).  -1 for arguments that a product refuses. */
+int mc_spmm_default_config(int lhs_bits, int rhs_bits, mc_signedness sign, int m_vec, int vec_length, int n, int k,
                            int row_slots);
-/* SpMM with the default tile for rows of row_slots nonzero vectors on average. */
+/* SpMM with the default tile for rows of row_slots slots on average. */
 mc_status mc_spmm_run_rows(int lhs_bits, int rhs_bits, mc_signedness sign, int row_slots, int m_vec,
                            int vec_length, int n, int k, const int *row_indices,
                            const int *row_offsets, const int *column_indices, const int *values,
                            const int *rhs_matrix, int *output_matrix, hipStream_t stream);
-/* Generic SpMM with an explicit config index (-1: the default for the shape).  (lhs_bits, rhs_bits) in {(8,8), (12,8), (16,8), (16,16),
- * (4,4), (8,4), (12,4), (16,4)}. */
+/* Generic SpMM with an explicit config index (-1: the default for the shape).
+ * (lhs_bits, rhs_bits) in {(8,8), (12,8), (16,8), (16,16), (4,4), (8,4),
+ * (12,4), (16,4)}. */
 mc_status mc_spmm_run(int lhs_bits, int rhs_bits, mc_signedness sign, int config, int m_vec,
                       int vec_length, int n, int k, const int *row_indices,
                       const int *row_offsets, const int *column_indices, const int *values,

@@ -34,7 +34,7 @@ _SIGS = {
     "mc_last_hip_error": (_I, []),
     "mc_spmm_num_tile_configs": (_I, []),
     "mc_spmm_get_tile_config": (_I, [_I, _P]),
-    "mc_spmm_default_config": (_I, [_I, _I, _I, _I, _I, _I, _I]),
+    "mc_spmm_default_config": (_I, [_I, _I, _I, _I, _I, _I, _I, _I]),
     "mc_spmm_run_rows": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
     "mc_spmm_run": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P]),
     "mc_format_row_alignment": (_I, [_I, _I]),

@@ -14,9 +14,48 @@ int mfma_rows(int lhs_bits, int rhs_bits, bool sgn, int V) {
     return (lhs_bits / 4 - (sgn ? 1 : 0)) * V;
 }
 
-// row_slots: nonzero vectors per vector row on average, 0 where the caller does
-// not know.
-int default_config(int rhs_bits, int n, long long m_vec, int rows, int row_slots) {
+// Slots per vector row from which wide products take four dwords per lane
+// (config 24) instead of one and four waves per row (17).  Short rows do not:
+// their gathers cost less than the fewer waves and the store through LDS.
+// Measured on MI355X over 5000 shapes (256 to 4096 rows, K 256 to 8192, 2 to 16
+// tiles, 16 to 1600 slots, V = 2, 4, 8, every pair of 8- and 16-bit B): by this
+// rule 0.5 % above the better of the two on average, always 24 2.8, always 17
+// 7.8.  It rests on, us 17 / 24 at 32, 64, 128, 256, 400 slots:
+// * the launch: L8-R8, V = 8, K = 1024, 1024 rows, N = 1024 9.3 / 10.0, 10.3 /
+//   11.4, 12.7 / 13.5, 20.5 / 20.3, 29.6 / 26.3; N = 4096 26.9 / 26.9, 32.4 /
+//   31.8, 41.0 / 40.2, 77.8 / 64.6, 117 / 85; few MFMA rows to recombine (V = 2),
+//   N = 2048 13.4 / 12.2, 15.4 / 14.2, 19.1 / 18.3;
+// * whole lines: where B's rows start off 64 bytes a wave's 4-byte gathers touch
+//   two lines for one, its 16-byte gathers five for four (1024 rows, K = 4096,
+//   L8-R8, V = 8, 256 slots: N = 1024 21.0 / 21.0, N = 976 23.7 / 21.6);
+// * the XCDs, which workgroups reach in turn: with G workgroups per row (the
+//   wide tile has two waves to one, 17 four) an XCD reads 1 / gcd(G, 8) of B.
+//   Where the wide tile's XCDs read more than 17's, and more than their L2
+//   holds, rows have to be longer (K = 4096, 256, 400, 800 slots: N = 3584 92.9 /
+//   111, 134 / 150, 252 / 226; N = 2560 60.4 / 70.7, 87.7 / 90.3, 163 / 127;
+//   16-bit B, N = 1792 84.8 / 102, 124 / 138, 241 / 203); where they read as much
+//   or less, rows may be shorter (N = 1792, 8-bit, 256 slots 48.5 / 32.7).
+int wide_least_slots(int rhs_bits, int n, int k, long long waves, int wide_tiles, int rows) {
+    constexpr long long kL2 = 4LL << 20;                        // of one XCD
+    const auto parts = [](int g) { return g & 1 ? 1 : g & 2 ? 2 : g & 4 ? 4 : 8; };   // gcd(g, 8)
+    const int here = parts((wide_tiles + 1) / 2), narrow = parts(wide_tiles);
+    const long long row_bytes = (long long)n * rhs_bits / 8, b_bytes = row_bytes * k;
+    const bool lines = row_bytes % 64 == 0;
+    const bool more = here < narrow && b_bytes / here > kL2;
+    if (more && lines) return 420;
+    if (rhs_bits == 16) return 0;                               // faster at every length
+    if (more) return 150;
+    int least = lines ? 300 : 150;
+    if (b_bytes > kL2 && here >= narrow) least = here > narrow ? 50 : least / 2;
+    if (rows <= 6 && waves >= (b_bytes <= kL2 ? 4096 : 8192)) return 0;
+    if (waves >= 16384) return least < 50 ? least : 50;
+    const int full = lines && b_bytes > kL2 ? 160 : 100;
+    return waves >= 8192 && full < least ? full : least;
+}
+
+// row_slots: slots per vector row on average, 0 where the caller does not know
+// (long rows then).
+int default_config(int rhs_bits, int n, int k, long long m_vec, int rows, int row_slots) {
     // Four dwords of 8- or 16-bit B per lane where the launch holds 2048 waves
     // of 16 * 4 dwords, two per workgroup (an odd tile's second wave included),
     // and a vector row is one MFMA row tile (two need 128 accumulators and
@@ -35,20 +74,14 @@ int default_config(int rhs_bits, int n, long long m_vec, int rows, int row_slots
     // / 14.1, 14.3 / 14.4).  Two tiles and four or five are faster from their
     // first column on (1024 rows: 260 20.0 / 13.7, 320 16.3 / 13.4, 772 37.4 /
     // 29.0, 1028 50.8 / 38.6; 512 rows: 772 19.9 / 17.3, 1028 27.9 / 21.7).
-    // Nor for short rows of 8-bit B, whose gathers cost less than the fewer
-    // waves and the store through LDS: the launch then has to be larger.  17 /
-    // this at 32, 96, 192, 256 and 400 slots per row: 1024 x 4096, N = 1024,
-    // L8-R8, V = 8 9.4 / 10.5, 11.9 / 13.2, 16.8 / 17.4, 21.0 / 21.0, 30.6 /
-    // 26.9; L16-R8, V = 4 12.4 / 13.1, 13.6 / 15.5, 17.5 / 19.2, 20.8 / 22.0,
-    // 30.1 / 27.1; N = 2048 15.2 / 17.4, 20.9 / 21.1, 33.1 / 31.5, 40.8 / 36.3,
-    // 60.1 / 47.0; N = 4096 (16384 waves) 30.4 / 31.8, 42.2 / 38.5, 63.9 / 53.7.
-    // 16-bit B is faster at every length (14.6 / 13.0, 16.1 / 16.0, 32.6 / 29.4).
+    // Nor for rows too short for it (wide_least_slots).
     if (rhs_bits != 4 && rows <= 16 && n % 4 == 0 && n >= 4 * (32 / rhs_bits)) {
         const int wide = 64 * (32 / rhs_bits);
         const int wide_tiles = (n + wide - 1) / wide;
         const long long waves = m_vec * 2 * ((wide_tiles + 1) / 2);
-        const int least = rhs_bits == 16 || waves >= 16384 ? 0 : waves >= 8192 ? 192 : 320;
-        if (waves >= 2048 && wide_tiles > 1 && wide_tiles != 3 && (row_slots == 0 || row_slots >= least)) return 24;
+        if (waves >= 2048 && wide_tiles > 1 && wide_tiles != 3 &&
+            (row_slots == 0 || row_slots >= wide_least_slots(rhs_bits, n, k, waves, wide_tiles, rows)))
+            return 24;
     }
     // One dword of B per lane and one k-block of gathers in flight per wave:
     // latency is hidden by more resident waves rather than deeper per-wave
@@ -118,7 +151,7 @@ mc_status spmm_entry(int lhs_bits, int rhs_bits, mc_signedness sign, int config,
     if (config < -1 || config >= kNumSpmmConfigs) return MC_EINVAL_ARG;
     // a batched launch fills the GPU with (row, tile) x batch workgroups
     const int rows = out16 ? 32 : mfma_rows(lhs_bits, rhs_bits, sign == MC_SIGNED, vec_length);
-    int cfg = config >= 0 ? config : default_config(rhs_bits, n, (long long)m_vec * batch, rows, row_slots);
+    int cfg = config >= 0 ? config : default_config(rhs_bits, n, k, (long long)m_vec * batch, rows, row_slots);
     if (!config_supported(cfg, rhs_bits)) return MC_EUNSUPPORTED;
     if (batch > 1 && kSpmmConfigs[cfg].kind == 1) return MC_EUNSUPPORTED;   // B-stationary: one matrix
     if (kSpmmConfigs[cfg].kind == 1 && !stationary_fits(cfg, n, k)) {
@@ -231,12 +264,12 @@ mc_status mc_spmm_get_tile_config(int index, mc_tile_config *out) {
     return MC_OK;
 }
 
-int mc_spmm_default_config(int lhs_bits, int rhs_bits, mc_signedness sign, int m_vec, int vec_length, int n,
+int mc_spmm_default_config(int lhs_bits, int rhs_bits, mc_signedness sign, int m_vec, int vec_length, int n, int k,
                            int row_slots) {
-    if (!mc::pair_supported(lhs_bits, rhs_bits) || !mc::valid_v(vec_length) || m_vec < 0 || n <= 0 ||
+    if (!mc::pair_supported(lhs_bits, rhs_bits) || !mc::valid_v(vec_length) || m_vec < 0 || n <= 0 || k < 0 ||
         n % (32 / rhs_bits) != 0 || row_slots < 0)
         return -1;
-    return mc::default_config(rhs_bits, n, m_vec, mc::mfma_rows(lhs_bits, rhs_bits, sign == MC_SIGNED, vec_length),
+    return mc::default_config(rhs_bits, n, k, m_vec, mc::mfma_rows(lhs_bits, rhs_bits, sign == MC_SIGNED, vec_length),
                               row_slots);
 }
 

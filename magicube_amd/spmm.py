@@ -84,12 +84,11 @@ def _check_device(tensors, what: str) -> None:
 
 
 def _row_slots(rhs_bits: int, m_vec: int, n: int, column_indices) -> int:
-    """Slots per vector row on average where the default tile depends on it
-    (short rows of 8-bit B over more columns than one wide tile), else 0."""
-    if rhs_bits != 8 or n <= 256 or not isinstance(column_indices, torch.Tensor):
+    """Slots per vector row on average where the default tile may depend on
+    them (8- and 16-bit B over more than 256 columns), else 0."""
+    if rhs_bits == 4 or n <= 256 or m_vec <= 0 or not isinstance(column_indices, torch.Tensor):
         return 0
-    slots = column_indices.numel() // max(m_vec, 1)
-    return max(slots, 1) if slots < 320 else 0
+    return max(column_indices.numel() // m_vec, 1)
 
 
 def wmma_spmm(lhs_bits: int, rhs_bits: int, m_vec: int, vec_length: int, n: int, k: int, row_indices,

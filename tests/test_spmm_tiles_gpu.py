@@ -52,7 +52,7 @@ def test_default_tile_of_long_rows(pair, V, signed, mclib):
     counts[:5] = (0, K, 65, 1, 0)
     widths = (132, 136, 256, 260, 264, 508, 512, 772, 776, 1028)
     product(pair, V, signed, m_vec, counts, widths, None, V)
-    tiles = {n: mclib.mc_spmm_default_config(*pair, 0 if signed else 1, m_vec, V, n, int(counts.mean())) for n in widths}
+    tiles = {n: mclib.mc_spmm_default_config(*pair, 0 if signed else 1, m_vec, V, n, K, int(counts.mean())) for n in widths}
     assert tiles[772] == tiles[1028] == 24
 
 
